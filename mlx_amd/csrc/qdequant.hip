@@ -15,19 +15,84 @@ __device__ __forceinline__ uint32_t row_code(const uint32_t* __restrict__ row, i
     return (uint32_t)(pair >> sh) & ((1u << bits) - 1u);
 }
 
-__global__ __launch_bounds__(256) void dequant_kernel(const uint32_t* __restrict__ wq,
-                                                      const void* __restrict__ sc,
-                                                      const void* __restrict__ bi,
-                                                      void* __restrict__ out, int N, int K,
-                                                      int gsize, int bits, int sb_dt, int out_dt) {
-    const size_t total = (size_t)N * K;
-    const int G = K / gsize, rw = (K * bits) >> 5;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-         i += (size_t)gridDim.x * blockDim.x) {
-        const int n = (int)(i / K), k = (int)(i - (size_t)n * K);
-        const uint32_t q = row_code(wq + (size_t)n * rw, k, bits);
-        const size_t gi = (size_t)n * G + k / gsize;
-        store_f(out, i, out_dt, fmaf(load_f(sc, gi, sb_dt), (float)q, load_f(bi, gi, sb_dt)));
+// Dequantizer.  Rows of codes, scales and outputs are each contiguous over the
+// whole [N, K] matrix (K is a multiple of the group size), so chunk t = the 8
+// codes 8t .. 8t+7 is BITS bytes at byte t * BITS of w_q, 8 outputs at element
+// 8t, and lies in one group.  Lane = chunk: a wave reads 64 * BITS contiguous
+// bytes and writes 1 KB of 16-bit (2 KB of f32) output in 16-byte stores.
+// Bound by HBM, by the output above all (117 of 150 MB at N = 14336, K = 4096,
+// 4-bit, f16); U chunks per lane, 256 apart, put U code and scale loads in
+// flight before the first store.  One lane per code, a 64-bit division per
+// code and 2-byte stores took 149 us at that size (1.0 TB/s).
+template <int SB>
+__device__ __forceinline__ float sb_at(const void* p, size_t i) {
+    if constexpr (SB == DT_F32) return static_cast<const float*>(p)[i];
+    else if constexpr (SB == DT_F16) return f16_to_f32(static_cast<const uint16_t*>(p)[i]);
+    else return bf16_to_f32(static_cast<const uint16_t*>(p)[i]);
+}
+
+// two fp32 values -> a packed pair of T, RNE (a scalar f16 cast of an fmaf
+// result could fuse into one rounding where the format rounds twice)
+template <int T>
+__device__ __forceinline__ uint32_t cvt_pk(float a, float b) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    if constexpr (T == DT_BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, b2));
+    else return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, h2));
+}
+
+template <int BITS, int SB, int OT, int U>
+__global__ __launch_bounds__(256) void dequant_kernel(const uint32_t* __restrict__ wq, const void* __restrict__ sc,
+                                                      const void* __restrict__ bi, void* __restrict__ out,
+                                                      size_t chunks, int gshift) {
+    typedef uint32_t o4 __attribute__((ext_vector_type(4)));
+    const size_t t0 = (size_t)blockIdx.x * (256 * U) + threadIdx.x;
+    uint32_t lo[U], hi[U];
+    float s[U], b[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const size_t t = t0 + 256 * u < chunks ? t0 + 256 * u : chunks - 1;
+        // the chunk's 8 BITS bits in the low end of hi:lo; where they are not
+        // whole words, from the two words they start in (up to 16 + 48 bits:
+        // the second word may lie past w_q, in its readable tail)
+        const size_t byte = t * BITS;
+        if constexpr (BITS == 2) {
+            lo[u] = reinterpret_cast<const uint16_t*>(wq)[t];
+        } else if constexpr (BITS == 4) {
+            lo[u] = wq[t];
+        } else {
+            const u32x2 v = *reinterpret_cast<const u32x2*>(wq + (byte >> 2));
+            const uint32_t sh = ((uint32_t)byte & 3u) * 8u;
+            lo[u] = BITS == 8 ? v.x : __builtin_amdgcn_alignbit(v.y, v.x, sh);
+            hi[u] = BITS == 8 ? v.y : v.y >> sh;
+        }
+        const size_t g = t >> gshift;
+        s[u] = sb_at<SB>(sc, g);
+        b[u] = sb_at<SB>(bi, g);
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const size_t t = t0 + 256 * u;
+        if (t >= chunks) return;
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            constexpr uint32_t mask = (1u << BITS) - 1u;
+            const int bit = i * BITS;
+            const uint32_t q = bit + BITS <= 32 ? (lo[u] >> bit) & mask
+                               : bit >= 32      ? (hi[u] >> (bit - 32)) & mask
+                                                : __builtin_amdgcn_alignbit(hi[u], lo[u], bit) & mask;
+            v[i] = fmaf(s[u], (float)q, b[u]);
+        }
+        o4* o = static_cast<o4*>(out) + t * (OT == DT_F32 ? 2 : 1);
+        if constexpr (OT == DT_F32) {
+            typedef float f4 __attribute__((ext_vector_type(4)));
+            o[0] = __builtin_bit_cast(o4, f4{v[0], v[1], v[2], v[3]});
+            o[1] = __builtin_bit_cast(o4, f4{v[4], v[5], v[6], v[7]});
+        } else {
+            o[0] = o4{cvt_pk<OT>(v[0], v[1]), cvt_pk<OT>(v[2], v[3]), cvt_pk<OT>(v[4], v[5]), cvt_pk<OT>(v[6], v[7])};
+        }
     }
 }
 
@@ -160,13 +225,55 @@ unsigned grid_for(size_t total) {
 
 }  // namespace
 
+namespace {
+// 4 chunks per lane where that still leaves every CU two blocks, else one
+template <int BITS, int SB, int OT>
+LuxStatus launch_dequant_t(const uint32_t* wq, const void* sc, const void* bi, void* out, size_t chunks, int gshift,
+                           hipStream_t st) {
+    if (chunks >= (size_t)512 * 1024) {
+        hipLaunchKernelGGL((dequant_kernel<BITS, SB, OT, 4>), dim3((unsigned)((chunks + 1023) / 1024)), dim3(256), 0,
+                           st, wq, sc, bi, out, chunks, gshift);
+    } else {
+        hipLaunchKernelGGL((dequant_kernel<BITS, SB, OT, 1>), dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st,
+                           wq, sc, bi, out, chunks, gshift);
+    }
+    return hipGetLastError() == hipSuccess ? LuxStatus::Ok : LuxStatus::Internal;
+}
+template <int BITS, int SB>
+LuxStatus launch_dequant_o(const uint32_t* wq, const void* sc, const void* bi, void* out, size_t chunks, int gshift,
+                           int out_dt, hipStream_t st) {
+    switch (out_dt) {
+    case DT_F32: return launch_dequant_t<BITS, SB, DT_F32>(wq, sc, bi, out, chunks, gshift, st);
+    case DT_F16: return launch_dequant_t<BITS, SB, DT_F16>(wq, sc, bi, out, chunks, gshift, st);
+    default: return launch_dequant_t<BITS, SB, DT_BF16>(wq, sc, bi, out, chunks, gshift, st);
+    }
+}
+template <int BITS>
+LuxStatus launch_dequant_b(const uint32_t* wq, const void* sc, const void* bi, void* out, size_t chunks, int gshift,
+                           int sb_dt, int out_dt, hipStream_t st) {
+    switch (sb_dt) {
+    case DT_F32: return launch_dequant_o<BITS, DT_F32>(wq, sc, bi, out, chunks, gshift, out_dt, st);
+    case DT_F16: return launch_dequant_o<BITS, DT_F16>(wq, sc, bi, out, chunks, gshift, out_dt, st);
+    default: return launch_dequant_o<BITS, DT_BF16>(wq, sc, bi, out, chunks, gshift, out_dt, st);
+    }
+}
+}  // namespace
+
 LuxStatus launch_dequantize(const uint32_t* wq, const void* scales, const void* biases, void* out,
                             int N, int K, int group_size, int bits, int sb_dtype, int out_dtype,
                             hipStream_t st) {
-    if ((size_t)N * K == 0) return LuxStatus::Ok;
-    hipLaunchKernelGGL(dequant_kernel, dim3(grid_for((size_t)N * K)), dim3(256), 0, st, wq, scales,
-                       biases, out, N, K, group_size, bits, sb_dtype, out_dtype);
-    return hipGetLastError() == hipSuccess ? LuxStatus::Ok : LuxStatus::Internal;
+    const size_t chunks = (size_t)N * K / 8;  // group sizes are 32, 64 and 128, so K % 8 == 0
+    if (chunks == 0) return LuxStatus::Ok;
+    const int gshift = group_size == 32 ? 2 : group_size == 64 ? 3 : 4;  // chunks per group, log2
+    switch (bits) {
+    case 2: return launch_dequant_b<2>(wq, scales, biases, out, chunks, gshift, sb_dtype, out_dtype, st);
+    case 3: return launch_dequant_b<3>(wq, scales, biases, out, chunks, gshift, sb_dtype, out_dtype, st);
+    case 4: return launch_dequant_b<4>(wq, scales, biases, out, chunks, gshift, sb_dtype, out_dtype, st);
+    case 5: return launch_dequant_b<5>(wq, scales, biases, out, chunks, gshift, sb_dtype, out_dtype, st);
+    case 6: return launch_dequant_b<6>(wq, scales, biases, out, chunks, gshift, sb_dtype, out_dtype, st);
+    case 8: return launch_dequant_b<8>(wq, scales, biases, out, chunks, gshift, sb_dtype, out_dtype, st);
+    default: return LuxStatus::NotSupported;
+    }
 }
 
 namespace {

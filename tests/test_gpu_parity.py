@@ -59,6 +59,24 @@ def test_dequantize_bit_exact(ctx, oracle, bits, sb):
 
 
 @pytest.mark.parametrize("bits", BITS)
+def test_dequantize_large_bit_exact(ctx, oracle, bits):
+    """Four chunks of 8 codes per lane (from 2^19 chunks on), the last block
+    and wave partial."""
+    from mlx_amd import runtime
+    O = oracle
+    N, K, gs = 1031, 4160, 32
+    rng = np.random.default_rng(bits)
+    w_q = rng.integers(0, 2**32, (N, K * bits // 32), dtype=np.uint32)
+    s, b = (rng.standard_normal((N, K // gs)).astype(np.float16).view(np.uint16) for _ in range(2))
+    for od in (F32, F16, BF16):
+        print(f"[case] dequant large bits={bits} out={od}", flush=True)
+        got = runtime.run_dequantize(ctx, w_q, s, b, K, gs, bits, F16, od)
+        want = O.dequantize(w_q, s, b, K, gs, bits, F16, od)
+        assert np.array_equal(got.view(np.uint16 if od else np.uint32),
+                              want.view(np.uint16 if od else np.uint32))
+
+
+@pytest.mark.parametrize("bits", BITS)
 @pytest.mark.parametrize("gs", [32, 64, 128])
 def test_quantize_bit_exact(ctx, oracle, bits, gs):
     """Codes, scales and biases bit-equal to the CPU quantizer, for f32 and
