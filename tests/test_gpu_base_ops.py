@@ -92,6 +92,14 @@ def test_matmul_bit_exact(ctx, M, K, N):
     assert np.array_equal(got.view(np.uint32), seq_matmul(a, b).view(np.uint32))
 
 
+@pytest.mark.parametrize("M,K,N", [(2040, 35, 2045), (1000, 33, 3001), (1000, 33, 1003), (500, 67, 1001),
+                                   (20, 131, 403), (1, 64, 4000), (1000, 1, 17)])
+def test_matmul_tiles_bit_exact(ctx, M, K, N):
+    """A shape per tile size (128 x 64, 64 x 64, 32 x 64, 32 x 32, 16 x 16),
+    ragged in M, K and N; K below, at and past a stage."""
+    test_matmul_bit_exact(ctx, M, K, N)
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 1), (3, 70), (64, 32), (129, 65)])
 def test_transpose_exact(ctx, rows, cols):
     a = np.random.default_rng(rows * cols).standard_normal((rows, cols)).astype(np.float32)
