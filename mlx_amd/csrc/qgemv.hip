@@ -31,6 +31,10 @@ static LuxStatus launch_mx_bits(const QmmArgs& a, hipStream_t st) {
 // kernels.  NotSupported: the generic kernel.
 LuxStatus launch_qgemv(const QmmArgs& args, hipStream_t st) {
     if (args.K % 64 != 0) return LuxStatus::NotSupported;
+    if (args.x_dtype == DT_F32) {
+        const LuxStatus s = launch_qgemm_f32(args, st);
+        if (s != LuxStatus::NotSupported) return s;
+    }
     // rows m0 .. m0 + mc - 1 of x and y
     auto rows = [&](int m0, int mc) {
         QmmArgs a = args;

@@ -1059,3 +1059,55 @@ def test_two_contexts_on_two_threads(oracle):
                     check_output(O, results[(tid, rep, i)], want, F32, f"thread {tid} rep {rep} case {i}")
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("bits", BITS)
+@pytest.mark.parametrize("M,K,N,gs,sb", [(17, 64, 1, 64, F32),      # one half step of K, one column
+                                         (32, 192, 127, 32, F16),   # a last half step, a full 32-row tile
+                                         (33, 1088, 129, 32, F32),  # two 32-row tiles, a second column tile
+                                         (65, 1152, 260, 128, BF16),  # a second row tile, odd steps over K parts
+                                         (64, 8256, 128, 64, F32)])  # many K parts, K % 128 == 64
+def test_f32_gemm(ctx, oracle, bits, M, K, N, gs, sb):
+    """f32 x on the bf16 matrix cores (three exact terms of x, exact codes)
+    against float64.  Every sum of 32 products and of K / 32 such sums is
+    rounded in f32, so an output is within (32 + K / 32 + 8) 2^-24 of the sum
+    of its terms' magnitudes."""
+    from mlx_amd import abi, runtime
+    O = oracle
+    assert ctx.kernel_name(M, K, N, gs, bits, F32, sb) == "qgemm_f32_kernel"
+    rng = np.random.default_rng(bits * 1000 + M)
+    q = rng.integers(0, 2**bits, (N, K))
+    w_q = rng.integers(0, 2**32, (N, K * bits // 32), dtype=np.uint32)
+    stream = np.unpackbits(w_q.view(np.uint8).reshape(N, -1), axis=1, bitorder="little")
+    q = (stream.reshape(N, K, bits) * (1 << np.arange(bits))).sum(-1).astype(np.float64)
+    s = O.from_f32(rng.uniform(0.5, 2, (N, K // gs)).astype(np.float32) * 0.01, sb)
+    b = O.from_f32(rng.standard_normal((N, K // gs)).astype(np.float32) * 0.02, sb)
+    x = (rng.standard_normal((M, K)) * 10.0 ** rng.integers(-3, 4, (M, 1))).astype(np.float32)
+    print(f"[case] f32 gemm M={M} K={K} N={N} bits={bits} gs={gs} sb={sb}", flush=True)
+    y = runtime.run_quantized_matmul(ctx, x, w_q, s, b, M, K, N, gs, bits, F32, sb, F32).astype(np.float64)
+    sf, bf = (np.repeat(O.to_f32(t, sb).astype(np.float64), gs, axis=1) for t in (s, b))
+    c = 2.0 ** (bits - 1)
+    want = x.astype(np.float64) @ (sf * q + bf).T
+    mag = np.abs(x).astype(np.float64) @ (sf * np.abs(q - c) + np.abs(bf + c * sf)).T
+    assert np.all(np.abs(y - want) <= (32 + K / 32 + 8) * 2.0**-24 * mag)
+
+
+def test_f32_gemm_special_values(ctx, oracle):
+    """An infinity or a NaN in a row of x reaches that row's outputs and no
+    other, and x of 2^120, all mantissa bits set, stays finite in its three
+    terms (times an 8-bit code it is just below the f32 range)."""
+    from mlx_amd import runtime
+    O = oracle
+    M, K, N = 20, 256, 130
+    x, w_q, s, b, _ = O.make_problem(M, K, N, 4, 64, F32, F32, seed=3)
+    clean = runtime.run_quantized_matmul(ctx, x, w_q, s, b, M, K, N, 64, 4, F32, F32, F32)
+    z = x.copy()
+    z[2, 5], z[7, 200], z[9, 0] = np.inf, np.nan, -np.inf
+    z[11, 77] = np.finfo(np.float32).max / 256
+    print("[case] f32 gemm special values", flush=True)
+    y = runtime.run_quantized_matmul(ctx, z, w_q, s, b, M, K, N, 64, 4, F32, F32, F32)
+    for m in (2, 7, 9):
+        assert not np.isfinite(y[m]).any()
+    assert np.isfinite(y[11]).all()
+    rest = [m for m in range(M) if m not in (2, 7, 9, 11)]
+    assert np.array_equal(y[rest], clean[rest])
