@@ -98,9 +98,10 @@ constexpr size_t kSplitWorkspaceBytes = (16u << 20) + 4096;
 // MFMA GEMM for M > 64 with each wave's W operand dequantized in its own
 // registers: 4/8-bit codes, f16/bf16 x, K % 1024 == 0; NotSupported otherwise
 LuxStatus launch_qgemm_rw(const QmmArgs& a, hipStream_t st);
-// MFMA GEMM for f32 activations, any code width, K % 64 == 0 (launch_qgemv
-// tries it first); NotSupported otherwise
-LuxStatus launch_qgemm_f32(const QmmArgs& a, hipStream_t st);
+// group-wise MFMA GEMM: any M, code width and type of x, K % 64 == 0, the
+// format's exact weights in f32 sums (the GEMV semantics); launch_qgemv takes
+// it for rows that would be split over launches
+LuxStatus launch_qgemm_grp(const QmmArgs& a, hipStream_t st);
 // MFMA GEMM for f16/bf16 activations; needs K % 64 == 0
 LuxStatus launch_qgemm(const QmmArgs& a, hipStream_t st);
 // generic one-thread-per-output kernel for shapes the tiled kernels reject

@@ -1,14 +1,16 @@
-// qgemm_f32.h -- MFMA GEMM for f32 activations (gfx950): any code width.
+// qgemm_grp.h -- group-wise MFMA GEMM (gfx950): any code width, type of x and
+// K % 64 == 0, with the GEMVs' semantics (the format's exact weights).
 //
 // y[m, n] = sum over groups g of  s (x . (q - C)) + (b + C s) sum_x,  s, b and
 // the sums per (n, g), C = 2^(BITS - 1): the format's definition regrouped as
-// the f32 GEMVs do it, with the inner products on the bf16 matrix cores and
+// the f32 GEMVs do it, with the inner products on the 16-bit matrix cores and
 // nothing rounded to 16 bits on the way:
-//  * a centred code (at most 8 bits) is a bf16 number exactly;
-//  * x is the sum of three bf16 numbers exactly: its leading 8 significant
-//    bits, the next 8 and the last 8, each by truncation (so the first never
-//    rounds up to infinity; below 2^-109 the third underflows);
-//  * a product of the two has at most 16 bits and is exact in the f32
+//  * a centred code (at most 8 bits) is a bf16 and an f16 number exactly;
+//  * 16-bit x goes in as it is; f32 x is the sum of three bf16 numbers
+//    exactly: its leading 8 significant bits, the next 8 and the last 8, each
+//    by truncation (so the first never rounds up to infinity; below 2^-109 the
+//    third underflows);
+//  * a product of the two has at most 19 bits and is exact in the f32
 //    accumulator, which is started afresh for every group and then scaled
 //    into the f32 sums of y.
 // An f32 FMA chain would round once per k; this rounds the partial sums of
@@ -29,13 +31,13 @@
 // next step's x is split into the three planes of the other LDS stage, with
 // its sums over 32 k, and the next codes are copied there; then the x and
 // codes of the step after that are loaded into the registers these leave; one
-// barrier.  (Two or three steps of loads in flight measured the same.)  Scales come in windows
-// of 32 bytes per column, 2 to 16 steps.  (Lanes that loaded their own
-// columns' codes and scales straight into registers touched 1000 cache lines
-// a step and took 1.5 times as long.)
+// barrier.  (Two or three steps of loads in flight measured the same.)
+// Scales come in windows of 32 bytes per column, 2 to 16 steps.  (Lanes that
+// loaded their own columns' codes and scales straight into registers touched
+// 1000 cache lines a step and took 1.5 times as long.)
 //
-// LDS: two stages of x, each three planes of 32 MT rows x 128 k bf16 (256
-// bytes a row; 16-byte chunk ch of row r at position ch ^ (r & 15): the
+// LDS: two stages of x, each one or (f32) three planes of 32 MT rows x 128 k
+// in 16 bits (256 bytes a row; 16-byte chunk ch of row r at position ch ^ (r & 15): the
 // fragment reads, 32 rows at one chunk, hit all banks evenly) and the sums of
 // x, [32 k][row]; two stages of codes, 16 BITS bytes a column; two scale
 // windows.  Column rows are padded so that 32 columns spread over the banks.
@@ -51,7 +53,7 @@
 #include "qsplit.h"
 
 namespace lxq {
-namespace f32g {
+namespace grp {
 
 // the kernel's lambdas hold register arrays: one left as a call would put them
 // in memory
@@ -59,6 +61,7 @@ namespace f32g {
 
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f4g __attribute__((ext_vector_type(4), aligned(4)));  // x and y may be dword-aligned only
@@ -69,11 +72,11 @@ typedef uint32_t u4h __attribute__((ext_vector_type(4), aligned(2)));  // scale 
 constexpr int BN = 128, BK = 128, kThreads = 512;
 constexpr int kRowBytes = BK * 2;  // one plane's row of a step
 
-template <int MT, int BITS>
+template <int MT, int BITS, int P>
 struct Lds {
     static constexpr int BM = 32 * MT;
     static constexpr int kPlane = BM * kRowBytes;
-    static constexpr int kSums = 3 * kPlane;               // [4][BM] f32
+    static constexpr int kSums = P * kPlane;               // [4][BM] f32
     static constexpr int kStage = kSums + 4 * BM * 4;
     static constexpr int kCodeRow = 16 * BITS + 16;
     static constexpr int kCodes = 2 * kStage;              // 2 x [128 columns]
@@ -82,13 +85,20 @@ struct Lds {
     static constexpr int kScales = kCodes + 2 * BN * kCodeRow;
     static constexpr int kOut = BN + 4;                    // floats per row of the output tile
     static constexpr int kTile = BM * kOut * 4;            // two of them at the end (pairs of K parts)
-    static constexpr int kBytes = kScales + 2 * kWindow;
-    static_assert(2 * kTile <= kBytes && kBytes <= 160 * 1024, "LDS");
+    static constexpr int kLoop = kScales + 2 * kWindow;
+    static constexpr int kBytes = kLoop > 2 * kTile ? kLoop : 2 * kTile;
+    static_assert(kBytes <= 160 * 1024, "LDS");
 };
 
+// f32 x runs on the bf16 units, like bf16
+template <int TX>
 __device__ __forceinline__ f32x16 mfma(const u4& a, const u4& b, const f32x16& c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
-                                                  0, 0);
+    if constexpr (TX == DT_F16)
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
+                                                     0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
+                                                      0, 0, 0);
 }
 
 // the top bit of every code that ends in word i of a run of 16 codes: codes
@@ -104,36 +114,45 @@ constexpr uint32_t top_bits(int i) {
 }
 
 // codes 8 j .. 8 j + 7 of the words w (top bits flipped; j a compile-time
-// constant after unrolling) as four packed pairs of bf16
-template <int BITS>
-__device__ __forceinline__ u4 bf16_codes8(const uint32_t* w, int j) {
-    uint32_t q[8];
+// constant after unrolling) as four packed pairs of the matrix type (both hold
+// every q - C exactly)
+template <int BITS, int TX>
+__device__ __forceinline__ u4 codes8(const uint32_t* w, int j) {
+    float q[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
         const int bit = (8 * j + i) * BITS, wi = bit >> 5, sh = bit & 31;
         const bool straddle = sh + BITS > 32;
         const uint32_t v = straddle ? __builtin_amdgcn_alignbit(w[straddle ? wi + 1 : wi], w[wi], sh) : w[wi];
-        q[i] = __float_as_uint((float)(int)__builtin_amdgcn_sbfe((int)v, straddle ? 0 : sh, BITS));
+        q[i] = (float)(int)__builtin_amdgcn_sbfe((int)v, straddle ? 0 : sh, BITS);
     }
     u4 r;
 #pragma unroll
-    for (int i = 0; i < 4; i++) r[i] = __builtin_amdgcn_perm(q[2 * i + 1], q[2 * i], 0x07060302u);
+    for (int i = 0; i < 4; i++) {
+        if constexpr (TX == DT_F16)
+            r[i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(q[2 * i], q[2 * i + 1]));
+        else
+            r[i] = __builtin_amdgcn_perm(__float_as_uint(q[2 * i + 1]), __float_as_uint(q[2 * i]), 0x07060302u);
+    }
     return r;
 }
 
-// BITS: code width; SBF: f32 scales (else 16-bit ones, sb_dt says which); MT:
+// BITS: code width; TX: type of x; SBF: f32 scales (else 16-bit ones, sb_dt says which); MT:
 // 32-row tiles
-template <int BITS, bool SBF, int MT>
-__global__ __launch_bounds__(kThreads, 1) void qgemm_f32_kernel(
-    const float* __restrict__ x, const uint32_t* __restrict__ wq, const void* __restrict__ scales,
+template <int BITS, int TX, bool SBF, int MT>
+__global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
+    const void* __restrict__ x, const uint32_t* __restrict__ wq, const void* __restrict__ scales,
     const void* __restrict__ biases, void* __restrict__ y, int M, int K, int N, int gshift, int sb_dt, Epilogue ep,
     int mtiles, int tiles, int parts, void* __restrict__ ws) {
-    using L = Lds<MT, BITS>;
+    constexpr int P = TX == DT_F32 ? 3 : 1;       // planes of x
+    using L = Lds<MT, BITS, P>;
     constexpr int BM = L::BM, NT = 2;
+    constexpr int XE = TX == DT_F32 ? 4 : 8;      // k per 16-byte load of x
     constexpr int WL = (BITS + 1) / 2;            // code words per lane, tile and step: 16 codes
-    constexpr int XL = BM * BK / 4 / kThreads;    // 16-byte loads of x per thread and step
+    constexpr int XL = BM * BK / XE / kThreads;   // 16-byte loads of x per thread and step
     constexpr int CL = (BITS + 3) / 4;            // 16-byte loads of codes per thread and step
-    constexpr int XR = kThreads / 32;             // rows per pass of x loads
+    constexpr int XC = BK / XE;                   // loads per row of x
+    constexpr int XR = kThreads / XC;             // rows per pass of x loads
     constexpr int kSb = SBF ? 4 : 2;
     constexpr float C = (float)(1 << (BITS - 1));
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -146,12 +165,13 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_f32_kernel(
     const int steps = (K + BK - 1) / BK;
     const int s0 = (int)((long long)steps * part / parts), s1 = (int)((long long)steps * (part + 1) / parts);
 
-    // x: thread t loads 4 k (chunk t % 32) of rows t / 32, + XR, ...; rows past
-    // M re-read the last (never stored), k past K are zeros
-    const int xc = tid & 31, xr = tid >> 5;
-    const float* xp[XL];
+    // x: thread t loads 16 bytes (chunk t % XC) of rows t / XC, + XR, ...; rows
+    // past M re-read the last (never stored), k past K are zeros
+    const int xc = tid % XC, xr = tid / XC;
+    const uint8_t* xp[XL];
 #pragma unroll
-    for (int i = 0; i < XL; i++) xp[i] = x + (size_t)min(m0 + xr + XR * i, M - 1) * K;
+    for (int i = 0; i < XL; i++)
+        xp[i] = static_cast<const uint8_t*>(x) + (size_t)min(m0 + xr + XR * i, M - 1) * K * (16 / XE);
     // codes: chunk q = t + 512 i of the block's 128 BITS: column q / BITS, 16
     // bytes q % BITS of its step (columns past N re-read the last; a half
     // step at the end of K reads on into the next row or the readable tail)
@@ -178,12 +198,13 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_f32_kernel(
     };
 
     struct Raw {
-        f4 x[XL];
+        u4 x[XL];
         u4 c[CL];
     };
     auto load = [&](Raw& o, int s) LXQ_INLINE {
 #pragma unroll
-        for (int i = 0; i < XL; i++) o.x[i] = *reinterpret_cast<const f4g*>(xp[i] + min(s * BK + 4 * xc, K - 4));
+        for (int i = 0; i < XL; i++)
+            o.x[i] = *reinterpret_cast<const u4h*>(xp[i] + (size_t)min(s * BK + XE * xc, K - XE) * (16 / XE));
 #pragma unroll
         for (int i = 0; i < CL; i++) o.c[i] = *reinterpret_cast<const u4g*>(cp[i] + (size_t)s * (16 * BITS));
     };
@@ -193,35 +214,46 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_f32_kernel(
         for (int i = 0; i < CL; i++)
             if (BITS % 4 == 0 || tid + kThreads * i < BN * BITS) *reinterpret_cast<u4*>(d + cd[i]) = o.c[i];
     };
-    // load i of step s into the three planes of stage st; the sum over the
-    // thread's 4 k.  FIX: an infinity's residue (inf - inf) is 0; a NaN's
-    // stays NaN
+    // load i of step s into the planes of stage st; the sum over the thread's
+    // XE k.  fix: an infinity's residue (inf - inf) is 0; a NaN's stays NaN
     auto split = [&](const Raw& o, int s, int i, uint8_t* st, float& big, auto fix) LXQ_INLINE {
-        f4 v = o.x[i];
-        if ((s + 1) * BK > K && s * BK + 4 * xc >= K) v = f4{0.f, 0.f, 0.f, 0.f};
-        big = fmaxf(fmaxf(big, fabsf(v.x)), fabsf(v.y));
-        big = fmaxf(fmaxf(big, fabsf(v.z)), fabsf(v.w));
-        uint32_t p[3][4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            p[0][e] = __float_as_uint(v[e]) & 0xffff0000u;
-            float r = v[e] - __uint_as_float(p[0][e]);
-            if constexpr (decltype(fix)::value) r = __builtin_isinf(v[e]) ? 0.f : r;
-            p[1][e] = __float_as_uint(r) & 0xffff0000u;
-            p[2][e] = __float_as_uint(r - __uint_as_float(p[1][e]));
-        }
+        u4 v = o.x[i];
+        if ((s + 1) * BK > K && s * BK + XE * xc >= K) v = u4{0u, 0u, 0u, 0u};
         const int row = xr + XR * i;
-        uint8_t* d = st + row * kRowBytes + (((xc >> 1) ^ (row & 15)) << 4) + (xc & 1) * 8;
+        uint8_t* d = st + row * kRowBytes;
+        if constexpr (TX == DT_F32) {
+            d += (((xc >> 1) ^ (row & 15)) << 4) + (xc & 1) * 8;
+            uint32_t p[3][4];
+            float f[4];
 #pragma unroll
-        for (int q = 0; q < 3; q++)
-            *reinterpret_cast<u2*>(d + q * L::kPlane) = u2{__builtin_amdgcn_perm(p[q][1], p[q][0], 0x07060302u),
-                                                           __builtin_amdgcn_perm(p[q][3], p[q][2], 0x07060302u)};
-        return (v.x + v.y) + (v.z + v.w);
+            for (int e = 0; e < 4; e++) {
+                f[e] = __uint_as_float(v[e]);
+                big = fmaxf(big, fabsf(f[e]));
+                p[0][e] = v[e] & 0xffff0000u;
+                float r = f[e] - __uint_as_float(p[0][e]);
+                if constexpr (decltype(fix)::value) r = __builtin_isinf(f[e]) ? 0.f : r;
+                p[1][e] = __float_as_uint(r) & 0xffff0000u;
+                p[2][e] = __float_as_uint(r - __uint_as_float(p[1][e]));
+            }
+#pragma unroll
+            for (int q = 0; q < 3; q++)
+                *reinterpret_cast<u2*>(d + q * L::kPlane) = u2{__builtin_amdgcn_perm(p[q][1], p[q][0], 0x07060302u),
+                                                               __builtin_amdgcn_perm(p[q][3], p[q][2], 0x07060302u)};
+            return (f[0] + f[1]) + (f[2] + f[3]);
+        } else {
+            *reinterpret_cast<u4*>(d + ((xc ^ (row & 15)) << 4)) = v;
+            float f[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                f[e] = TX == DT_F16 ? f16_to_f32(v[e] & 0xffffu) + f16_to_f32(v[e] >> 16)
+                                    : bf16_to_f32(v[e]) + __uint_as_float(v[e] & 0xffff0000u);
+            return (f[0] + f[1]) + (f[2] + f[3]);
+        }
     };
     // after the splits of a step: the rare step that holds an infinity is
-    // split again; the sums over 32 k (8 lanes)
+    // split again; the sums over 32 k (32 / XE lanes)
     auto finish = [&](const Raw& o, int s, float (&sum)[XL], uint8_t* st, float big) LXQ_INLINE {
-        if (__any(big == __builtin_inff())) {
+        if (TX == DT_F32 && __any(big == __builtin_inff())) {
 #pragma unroll
             for (int i = 0; i < XL; i++) split(o, s, i, st, big, std::true_type{});
         }
@@ -229,12 +261,15 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_f32_kernel(
         for (int i = 0; i < XL; i++) sum[i] += dpp_f<0xB1>(sum[i]);
 #pragma unroll
         for (int i = 0; i < XL; i++) sum[i] += dpp_f<0x4E>(sum[i]);
+        if constexpr (TX == DT_F32) {
 #pragma unroll
-        for (int i = 0; i < XL; i++) sum[i] += dpp_f<0x141>(sum[i]);
-        if ((xc & 7) == 0) {
+            for (int i = 0; i < XL; i++) sum[i] += dpp_f<0x141>(sum[i]);
+        }
+        constexpr int LG = 32 / XE;
+        if (xc % LG == 0) {
 #pragma unroll
             for (int i = 0; i < XL; i++)
-                *reinterpret_cast<float*>(st + L::kSums + ((xc >> 3) * BM + xr + XR * i) * 4) = sum[i];
+                *reinterpret_cast<float*>(st + L::kSums + (xc / LG * BM + xr + XR * i) * 4) = sum[i];
         }
     };
     auto sb_f = [&](const uint8_t* p) LXQ_INLINE {
@@ -290,17 +325,17 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_f32_kernel(
         for (int j = 0; j < 2; j++) {
             // sub-step j: k 16 h + 8 j .. +8 of the wave's 32 (chunk of the row)
             const int ch = 4 * kg + 2 * h + j;
-            u4 a[MT][3], b[NT];
+            u4 a[MT][P], b[NT];
 #pragma unroll
             for (int i = 0; i < MT; i++)
 #pragma unroll
-                for (int q = 0; q < 3; q++)
+                for (int q = 0; q < P; q++)
                     a[i][q] = *reinterpret_cast<const u4*>(st + q * L::kPlane + (32 * i + c) * kRowBytes +
                                                            ((ch ^ (c & 15)) << 4));
 #pragma unroll
-            for (int t = 0; t < NT; t++) b[t] = bf16_codes8<BITS>(w[t], j);
+            for (int t = 0; t < NT; t++) b[t] = codes8<BITS, TX>(w[t], j);
 #pragma unroll
-            for (int q = 0; q < 3; q++)
+            for (int q = 0; q < P; q++)
 #pragma unroll
                 for (int i = 0; i < MT; i++)
 #pragma unroll
@@ -309,9 +344,9 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_f32_kernel(
                             f32x16 z;
 #pragma unroll
                             for (int v = 0; v < 16; v++) z[v] = 0.f;
-                            g[i][t] = mfma(a[i][q], b[t], z);
+                            g[i][t] = mfma<TX>(a[i][q], b[t], z);
                         } else {
-                            g[i][t] = mfma(a[i][q], b[t], g[i][t]);
+                            g[i][t] = mfma<TX>(a[i][q], b[t], g[i][t]);
                         }
                     }
 #pragma unroll
@@ -371,13 +406,14 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_f32_kernel(
         }
         __syncthreads();
     }
-    // thread: 4 columns (16 bytes) of rows tid / 32 + XR i
+    // thread: 4 columns (16 bytes) of rows tid / 32 + 16 i
+    const int oc = 4 * (tid & 31), orow = tid >> 5;
     constexpr int kVec = BM * BN / 4 / kThreads;
     constexpr uint32_t kSlot = BM * BN * 4;
     f4 o[kVec];
 #pragma unroll
     for (int i = 0; i < kVec; i++) {
-        const float* d = reinterpret_cast<const float*>(lds) + (xr + XR * i) * L::kOut + 4 * xc;
+        const float* d = reinterpret_cast<const float*>(lds) + (orow + 16 * i) * L::kOut + oc;
         o[i] = *reinterpret_cast<const f4*>(d) + *reinterpret_cast<const f4*>(d + L::kTile / 4);
     }
     if (parts > 1) {
@@ -419,7 +455,7 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_f32_kernel(
     const bool plain = ep.bias == nullptr && ep.act == ACT_NONE && ep.out_dt == DT_F32 && N % 4 == 0;
 #pragma unroll
     for (int i = 0; i < kVec; i++) {
-        const int m = m0 + xr + XR * i, n = n0 + 4 * xc;
+        const int m = m0 + orow + 16 * i, n = n0 + oc;
         if (m >= M) continue;
         if (plain) {
             if (n < N) *reinterpret_cast<f4g*>(static_cast<float*>(y) + (size_t)m * N + n) = o[i];
@@ -431,16 +467,18 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_f32_kernel(
     }
 }
 
-template <int BITS, bool SBF, int MT>
+template <int BITS, int TX, bool SBF, int MT>
 LuxStatus launch_t(const QmmArgs& a, hipStream_t st) {
-    using L = Lds<MT, BITS>;
-    if (planned(a, "qgemm_f32_kernel")) return LuxStatus::Ok;
-    auto kern = qgemm_f32_kernel<BITS, SBF, MT>;
+    using L = Lds<MT, BITS, TX == DT_F32 ? 3 : 1>;
+    if (planned(a, "qgemm_grp_kernel")) return LuxStatus::Ok;
+    auto kern = qgemm_grp_kernel<BITS, TX, SBF, MT>;
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, L::kBytes);
     if (attr != hipSuccess) return LuxStatus::Internal;
     const int mtiles = (a.M + L::BM - 1) / L::BM, ntiles = (a.N + BN - 1) / BN;
-    const int tiles = mtiles * ntiles, steps = (a.K + BK - 1) / BK;
+    const size_t all = (size_t)mtiles * ntiles;
+    if (all >= (1ull << 31)) return LuxStatus::NotSupported;
+    const int tiles = (int)all, steps = (a.K + BK - 1) / BK;
     // K parts until there is a block per CU, at least two steps each, within
     // the workspace
     int parts = 1;
@@ -453,17 +491,34 @@ LuxStatus launch_t(const QmmArgs& a, hipStream_t st) {
         if (parts < 1) parts = 1;
     }
     const int gshift = a.group_size == 32 ? 5 : a.group_size == 64 ? 6 : 7;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * parts)), dim3(kThreads), L::kBytes, st,
-                       static_cast<const float*>(a.x), a.wq, a.scales, a.biases, a.y, a.M, a.K, a.N, gshift,
-                       a.sb_dtype, a.epi(), mtiles, tiles, parts, a.ws);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * parts)), dim3(kThreads), L::kBytes, st, a.x, a.wq, a.scales,
+                       a.biases, a.y, a.M, a.K, a.N, gshift, a.sb_dtype, a.epi(), mtiles, tiles, parts, a.ws);
     return hipGetLastError() == hipSuccess ? LuxStatus::Ok : LuxStatus::Internal;
 }
 
-template <int BITS>
-LuxStatus launch_b(const QmmArgs& a, hipStream_t st) {
-    if (a.sb_dtype == DT_F32) return a.M <= 32 ? launch_t<BITS, true, 1>(a, st) : launch_t<BITS, true, 2>(a, st);
-    return a.M <= 32 ? launch_t<BITS, false, 1>(a, st) : launch_t<BITS, false, 2>(a, st);
+template <int BITS, int TX>
+LuxStatus launch_x(const QmmArgs& a, hipStream_t st) {
+    if (a.sb_dtype == DT_F32)
+        return a.M <= 32 ? launch_t<BITS, TX, true, 1>(a, st) : launch_t<BITS, TX, true, 2>(a, st);
+    return a.M <= 32 ? launch_t<BITS, TX, false, 1>(a, st) : launch_t<BITS, TX, false, 2>(a, st);
 }
 
-}  // namespace f32g
+template <int TX>
+LuxStatus launch_b(const QmmArgs& a, hipStream_t st) {
+    switch (a.bits) {
+    case 2: return launch_x<2, TX>(a, st);
+    case 3: return launch_x<3, TX>(a, st);
+    case 4: return launch_x<4, TX>(a, st);
+    case 5: return launch_x<5, TX>(a, st);
+    case 6: return launch_x<6, TX>(a, st);
+    case 8: return launch_x<8, TX>(a, st);
+    default: return LuxStatus::NotSupported;
+    }
+}
+
+extern template LuxStatus launch_b<DT_F32>(const QmmArgs&, hipStream_t);
+extern template LuxStatus launch_b<DT_F16>(const QmmArgs&, hipStream_t);
+extern template LuxStatus launch_b<DT_BF16>(const QmmArgs&, hipStream_t);
+
+}  // namespace grp
 }  // namespace lxq

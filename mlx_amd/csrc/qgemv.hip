@@ -25,16 +25,58 @@ static LuxStatus launch_mx_bits(const QmmArgs& a, hipStream_t st) {
     }
 }
 
+// Whether f32 x runs on the group-wise GEMM: from 9 rows where the K-split
+// whole-line kernel takes 4 rows a launch, from 5 where every row is a launch
+// of its own (3/5/6-bit codes, K it does not divide).  g64, f32 scales, 4-bit,
+// us per launch against those kernels: K = N = 4096, M = 5 / 8 / 16 / 32 / 64
+// 12.7 / 12.7 / 13.0 / 13.2 / 19.5 against 10.9 / 13.2 / 26.3 / 53.3 / 108; K
+// = 4096, N = 14336, M = 8 / 16 / 128 27.8 / 27.1 / 72.5 against 30.2 / 60.2 /
+// 470; 3-bit K = 14336, N = 4096, M = 16 31 against 145; 5-bit K = 640, N =
+// 1000, M = 16 10.4 against 66.7.  The whole-line kernel keeps its class of up
+// to 16 rows of 3/5/6-bit codes at K <= 4096.
+static bool grp_f32(const QmmArgs& a) {
+    const bool irregular = a.bits == 3 || a.bits == 5 || a.bits == 6;
+    const int mx_step = 16 * (a.K > 8192 ? 16 : a.K > 4096 ? 8 : 4);
+    const bool rows = irregular || a.K > 16384 || a.K % mx_step != 0;
+    return a.M >= (!rows ? 9 : irregular && a.K <= 4096 ? 17 : 5);
+}
+
+// Whether 16-bit x that no M-wide kernel takes runs on the group-wise GEMM
+// instead of launches of 4 rows (K <= 4096) or 2 (K > 4096).  g64, bf16, us
+// per launch:
+//  * K > 4096, three launches or more: K = 4160, N = 4096 M = 5 / 8 / 12 / 32
+//    12.3 / 12.4 / 12.7 / 13.4 against 20.0 / 25.9 / 38.8 / 103; K = 9856, N =
+//    1035, 8-bit M = 1303 109 against 4170.  Two: 3-bit K = 5120, N = 13824,
+//    M = 4 33.0 against 40.9, 5-bit K = 6144, N = 1024 12.8 against 11.2: from
+//    4096 columns; M = 3 33.0 against 35.2, 19.4 against 18.3 (5-bit, K =
+//    8256): not.
+//  * K <= 4096, three launches or more: K = 832, N = 1000, 3-bit M = 12 9.4
+//    against 16.0; K = 3200, N = 1000 M = 1000 27.7 against 1344.  Two: 8-bit
+//    codes (K = 1920, N = 8193 M = 5 11.4 against 14.9; N = 1000 M = 8 8.3
+//    against 11.1); the others stay (K = N = 4096, 3-bit M = 6 12.8 against
+//    9.7).
+//  * Up to 8 rows and 320 columns (three tiles: K in as many parts as CUs, the
+//    last of which adds them all) stay with the launches.
+// Shapes the GEMMs take (K % 256 == 0) come here with more rows only when the
+// GEMV is asked for by name, and keep its kernels (f32 scales of groups of 32
+// at 6 and 8 bits they do not take).
+constexpr int kGrpCols = 320;
+
+static bool grp_rows(const QmmArgs& a) {
+    if (a.x_dtype == DT_F32) return false;
+    if (a.M <= 8 && a.N <= kGrpCols) return false;
+    if (a.K > 4096) return a.M >= 5 || (a.M == 4 && a.N >= 4096);
+    if (a.M <= 8) return a.M >= 5 && a.bits == 8;
+    return a.K % 256 != 0 || (a.sb_dtype == DT_F32 && a.group_size == 32 && a.bits >= 6);
+}
+
 // Rows of x that no kernel takes whole are split over launches: four rows
-// of 16-bit x per launch of the stream kernel (K <= 4096), two per launch of
-// the split-K kernel (K > 4096), one row of f32 x per launch of the M = 1
+// of 16-bit x per launch of the stream kernel (K <= 4096), two and one of the
+// split-K kernel (K > 4096), one row of f32 x per launch of the M = 1
 // kernels.  NotSupported: the generic kernel.
 LuxStatus launch_qgemv(const QmmArgs& args, hipStream_t st) {
     if (args.K % 64 != 0) return LuxStatus::NotSupported;
-    if (args.x_dtype == DT_F32) {
-        const LuxStatus s = launch_qgemm_f32(args, st);
-        if (s != LuxStatus::NotSupported) return s;
-    }
+    if (args.x_dtype == DT_F32 && grp_f32(args)) return launch_qgemm_grp(args, st);
     // rows m0 .. m0 + mc - 1 of x and y
     auto rows = [&](int m0, int mc) {
         QmmArgs a = args;
@@ -77,20 +119,20 @@ LuxStatus launch_qgemv(const QmmArgs& args, hipStream_t st) {
         const LuxStatus s = launch_qgemv_q4(args, st);
         if (s != LuxStatus::NotSupported) return s;
     }
-    // 5..8 rows of x, 16-bit x, 8192 < K <= 16384: rows 0..3 and the rest as
-    // two launches of the kernels above (the second finds W in the Infinity
-    // Cache) where the LDS-ring kernel does not take the shape (K % 1024 !=
-    // 0, 2-bit codes) or fills half the CUs (4-bit, N <= 4096; its 32-row
-    // blocks).  Same box, g64, N = 4096, M = 5 / 6 / 8, us per launch: K =
-    // 11008, 4-bit 32.3 / 35.5 / 46.8 -> 18.5 / 17.5 / 18.7 (split-K kernel
-    // before), 8-bit 37.8 / 41.1 / 54.1 -> 32.1 / 34.7 / 39.3; K = 14336,
-    // 2-bit 34.4 / 41.0 / 54.4 -> 23.1 / 25.0 / 29.5, 4-bit 25.4 / 25.5 /
-    // 25.4 -> 21.2 / 21.5 / 23.0 (LDS-ring kernel before).  Not taken: 8-bit
-    // at K = 14336 (27.4 -> 33.9..40.7) and 4-bit at N = 8192 (27.5 ->
-    // 37.8..44.9), where the LDS-ring kernel fills the CUs.
+    // 5..8 rows of x, 16-bit x, 8192 < K <= 16384, where the LDS-ring kernel
+    // does not take the shape (K % 1024 != 0, 2-bit codes) or fills half the
+    // CUs (4-bit, N <= 4096; its 32-row blocks): the group-wise GEMM; up to
+    // kGrpCols columns rows 0..3 and the rest as two launches of the kernels
+    // above.  Same box, g64, N = 4096, us per launch, against the two
+    // launches: K = 11008, 8-bit M = 5 / 8 17.3 / 17.4 against 33.8 / 43.9,
+    // 4-bit 18.2 / 18.2 against 18.0 / 18.6; K = 14336, 2-bit 21.3 / 21.3
+    // against 22.2 / 29.1 (N = 14336: 60 against 108), 4-bit M = 8 21.3
+    // against 23.2.  Not taken: 4-bit at N = 8192 (27.5 on the LDS-ring
+    // kernel, which fills the CUs there).
     if (args.M >= 5 && args.M <= 8 && args.x_dtype != DT_F32 && args.K > 8192 && args.K <= 16384 &&
         (args.bits == 2 || args.bits == 4 || args.bits == 8) &&
         (args.K % 1024 != 0 || args.bits == 2 || (args.bits == 4 && args.N <= 4096))) {
+        if (args.N > kGrpCols) return launch_qgemm_grp(args, st);
         const LuxStatus s = launch_qgemv(rows(0, 4), st);
         if (s != LuxStatus::Ok) return s;
         return launch_qgemv(rows(4, args.M - 4), st);
@@ -113,6 +155,7 @@ LuxStatus launch_qgemv(const QmmArgs& args, hipStream_t st) {
         const LuxStatus s = launch_qmm_skinny(args, st);
         if (s != LuxStatus::NotSupported) return s;
     }
+    if (grp_rows(args)) return launch_qgemm_grp(args, st);
     // f32 x, two rows or more, where the K-split whole-line kernel does not
     // run (3/5/6-bit codes; K > 16384; K not a whole number of its waves'
     // 16-code steps, launch_mx_b): one launch of the M = 1 kernels per
@@ -123,8 +166,7 @@ LuxStatus launch_qgemv(const QmmArgs& args, hipStream_t st) {
     // 3 / 4 / 8: 3-bit 35.6 / 45.6 / 68.3 / 133.4 -> 17.6 / 26.0 / 34.5 /
     // 68.0; 5-bit 56.5 / 72.0 / 114.9 / 224.2 -> 22.1 / 32.8 / 43.3 / 86.0;
     // 6-bit 57.0 / 70.2 / 116.4 / 227.5 -> 23.4 / 34.4 / 45.8 / 88.8 (N =
-    // 4096: 40-52 % less).  Every row is the same launch, so the gain holds
-    // at any M.
+    // 4096: 40-52 % less).  More rows: grp_f32.
     if (args.x_dtype == DT_F32 && args.M >= 2 &&
         (args.bits == 3 || args.bits == 5 || args.bits == 6 || args.K > 16384 ||
          args.K % (16 * (args.K > 8192 ? 16 : args.K > 4096 ? 8 : 4)) != 0)) {
@@ -142,9 +184,8 @@ LuxStatus launch_qgemv(const QmmArgs& args, hipStream_t st) {
         const LuxStatus s = launch_bits(args, st);
         if (s != LuxStatus::NotSupported) return s;
     }
-    // f32 x with more than 4 rows: chunks of 4 (a last single row on the
-    // M = 1 kernels) on the K-split whole-line kernel where it applies
-    // (M = 8, K = 4096, N = 14336, 4-bit: the row-run kernel took 126.9 us)
+    // f32 x, 5..8 rows: 4 and the rest (a single row on the M = 1 kernels) on
+    // the K-split whole-line kernel where it applies
     if (args.x_dtype == DT_F32 && args.M > 4) {
         for (int m0 = 0; m0 < args.M; m0 += 4) {
             const QmmArgs a = rows(m0, args.M - m0 < 4 ? args.M - m0 : 4);
@@ -154,14 +195,11 @@ LuxStatus launch_qgemv(const QmmArgs& args, hipStream_t st) {
             if (m0 + 4 >= args.M) return LuxStatus::Ok;
         }
     }
-    // 16-bit x, K > 4096, three rows or more that no kernel above took:
-    // pairs of rows on the split-K kernel (a last single row on the M = 1
-    // kernels) rather than a row-run kernel (since retired) in chunks of up to 4 rows, or
-    // the generic kernel where one row of x overflows its 64 KB staging.
-    // Same box, g64, us per launch: K = 5120, N = 13824, 3-bit, M = 3 / 4 /
-    // 8: 81.8 / 99.5 / 186.7 -> 36.3 / 41.8 / 82.6 (5/6-bit alike); K =
-    // 6144, N = 4096, M = 4: 36.0 -> 16.3; 4-bit K = 6656 40.6 -> 15.8; K =
-    // 28672, N = 8192, 3-bit M = 3 / 8: 17132 / 24198 -> 92.7 / 238.5
+    // 16-bit x, K > 4096, three rows or more that no kernel above took: pairs
+    // of rows on the split-K kernel (a last single row on the M = 1 kernels)
+    // rather than a row-run kernel (since retired) in chunks of up to 4 rows.
+    // Same box, g64, us per launch: K = 5120, N = 13824, 3-bit, M = 3: 81.8 ->
+    // 36.3 (5/6-bit alike); K = 28672, N = 8192, 3-bit M = 3: 17132 -> 92.7
     if (args.x_dtype != DT_F32 && args.K > 4096 && args.M > 2) {
         for (int m0 = 0; m0 < args.M; m0 += 2) {
             const LuxStatus s = launch_bits(rows(m0, args.M - m0 < 2 ? 1 : 2), st);

@@ -1061,34 +1061,36 @@ def test_two_contexts_on_two_threads(oracle):
         ctx.close()
 
 
+@pytest.mark.parametrize("xd", [F32, F16, BF16])
 @pytest.mark.parametrize("bits", BITS)
 @pytest.mark.parametrize("M,K,N,gs,sb", [(17, 64, 1, 64, F32),      # one half step of K, one column
                                          (32, 192, 127, 32, F16),   # a last half step, a full 32-row tile
                                          (33, 1088, 129, 32, F32),  # two 32-row tiles, a second column tile
                                          (65, 1152, 260, 128, BF16),  # a second row tile, odd steps over K parts
                                          (64, 8256, 128, 64, F32)])  # many K parts, K % 128 == 64
-def test_f32_gemm(ctx, oracle, bits, M, K, N, gs, sb):
-    """f32 x on the bf16 matrix cores (three exact terms of x, exact codes)
-    against float64.  Every sum of 32 products and of K / 32 such sums is
-    rounded in f32, so an output is within (32 + K / 32 + 8) 2^-24 of the sum
-    of its terms' magnitudes."""
-    from mlx_amd import abi, runtime
+def test_group_gemm(ctx, oracle, bits, M, K, N, gs, sb, xd):
+    """The group-wise GEMM (x and codes exact on the matrix cores; f32 x as
+    three exact terms) against float64, rows of x over nine decades (f16
+    subnormals among them).  Every sum of 32 products and of K / 32 such sums
+    is rounded in f32, so an f32 output is within (32 + K / 32 + 8) 2^-24 of
+    the sum of its terms' magnitudes."""
+    from mlx_amd import runtime
     O = oracle
-    assert ctx.kernel_name(M, K, N, gs, bits, F32, sb) == "qgemm_f32_kernel"
+    assert ctx.kernel_name(M, K, N, gs, bits, xd, sb, F32) == "qgemm_grp_kernel"
     rng = np.random.default_rng(bits * 1000 + M)
-    q = rng.integers(0, 2**bits, (N, K))
     w_q = rng.integers(0, 2**32, (N, K * bits // 32), dtype=np.uint32)
     stream = np.unpackbits(w_q.view(np.uint8).reshape(N, -1), axis=1, bitorder="little")
     q = (stream.reshape(N, K, bits) * (1 << np.arange(bits))).sum(-1).astype(np.float64)
     s = O.from_f32(rng.uniform(0.5, 2, (N, K // gs)).astype(np.float32) * 0.01, sb)
     b = O.from_f32(rng.standard_normal((N, K // gs)).astype(np.float32) * 0.02, sb)
-    x = (rng.standard_normal((M, K)) * 10.0 ** rng.integers(-3, 4, (M, 1))).astype(np.float32)
-    print(f"[case] f32 gemm M={M} K={K} N={N} bits={bits} gs={gs} sb={sb}", flush=True)
-    y = runtime.run_quantized_matmul(ctx, x, w_q, s, b, M, K, N, gs, bits, F32, sb, F32).astype(np.float64)
+    x = O.from_f32((rng.standard_normal((M, K)) * 10.0 ** rng.integers(-6, 4, (M, 1))).astype(np.float32), xd)
+    print(f"[case] group gemm M={M} K={K} N={N} bits={bits} gs={gs} sb={sb} x={xd}", flush=True)
+    y = runtime.run_quantized_matmul(ctx, x, w_q, s, b, M, K, N, gs, bits, xd, sb, F32).astype(np.float64)
+    xf = O.to_f32(x, xd).astype(np.float64)
     sf, bf = (np.repeat(O.to_f32(t, sb).astype(np.float64), gs, axis=1) for t in (s, b))
     c = 2.0 ** (bits - 1)
-    want = x.astype(np.float64) @ (sf * q + bf).T
-    mag = np.abs(x).astype(np.float64) @ (sf * np.abs(q - c) + np.abs(bf + c * sf)).T
+    want = xf @ (sf * q + bf).T
+    mag = np.abs(xf) @ (sf * np.abs(q - c) + np.abs(bf + c * sf)).T
     assert np.all(np.abs(y - want) <= (32 + K / 32 + 8) * 2.0**-24 * mag)
 
 
