@@ -90,11 +90,12 @@ LuxStatus launch_qgemm_sk(const QmmArgs& a, hipStream_t st);
 size_t qgemm_sk_workspace(int M, int K, int N, int bits, int x_dtype, size_t cap);
 // the workspace every caller of the GEMMs provides (a context's, or the
 // allocation-free entry point's static one): the same size everywhere, so
-// the same shape takes the same split, and the same result bits.  16 MiB of
-// partials: the split-K small-M GEMM's largest split (512 blocks of 32 KiB),
-// and the large GEMM's split last round (at most 128 tiles, one K half of
-// 128 KiB each).  The first KiB holds tile counters and flags.
-constexpr size_t kSplitWorkspaceBytes = (16u << 20) + 4096;
+// the same shape takes the same split, and the same result bits.  32 MiB of
+// partials: one 128 KiB tile of fp32 sums per CU (the K parts of the large
+// GEMMs; their split last round, at most 128 tiles of one K half each, and the
+// split-K small-M GEMM's largest split, 512 blocks of 32 KiB, need half).  The
+// first KiB holds tile counters and flags.
+constexpr size_t kSplitWorkspaceBytes = (32u << 20) + 4096;
 // MFMA GEMM for M > 64 with each wave's W operand dequantized in its own
 // registers: 4/8-bit codes, f16/bf16 x, K % 1024 == 0; NotSupported otherwise
 LuxStatus launch_qgemm_rw(const QmmArgs& a, hipStream_t st);

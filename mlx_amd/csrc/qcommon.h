@@ -49,13 +49,17 @@ __device__ __forceinline__ void store_f(void* p, size_t i, int dt, float v) {
     else reinterpret_cast<uint16_t*>(p)[i] = f32_to_bf16(v);
 }
 
-// the output stage (Epilogue, kernels.h) for column n, then the store
+// the output stage (Epilogue, kernels.h): the activation, and all of it for
+// column n, then the store
+__device__ __forceinline__ float apply_act(int act, float v) {
+    if (act == ACT_RELU) v = v < 0.f ? 0.f : v;
+    else if (act == ACT_SILU) v = v / (1.f + expf(-v));
+    else if (act == ACT_GELU) v = 0.5f * v * (1.f + erff(v * 0.70710678118654752f));
+    return v;
+}
 __device__ __forceinline__ float apply_epilogue(const Epilogue& e, size_t n, float v) {
     if (e.bias) v = v + load_f(e.bias, n, e.bias_dt);
-    if (e.act == ACT_RELU) v = v < 0.f ? 0.f : v;
-    else if (e.act == ACT_SILU) v = v / (1.f + expf(-v));
-    else if (e.act == ACT_GELU) v = 0.5f * v * (1.f + erff(v * 0.70710678118654752f));
-    return v;
+    return apply_act(e.act, v);
 }
 // EPI: the kernel instantiation that applies the output stage (else only
 // the store; out_dt is read from e in both)

@@ -41,8 +41,12 @@
 // and takes half as long; the two halves' fp32 sums meet in the workspace
 // (the second block to finish adds the first's partial tile to its own --
 // one fp32 addition per value, the same whichever finishes first -- and
-// stores y).
+// stores y).  Fewer than 129 tiles run in K parts (k_parts):
+// every part stores its fp32 tile, and a second launch adds them in part
+// order and stores y.
 #pragma once
+#include <algorithm>
+
 #include "kernels.h"
 #include "qcommon.h"
 #include "qsplit.h"
@@ -159,6 +163,11 @@ constexpr size_t lds_bytes() {
            (size_t)kPackSlots * pack_slot_bytes<BITS>() + 2 * (size_t)Win<GS, SB>::kSlotBytes;
 }
 constexpr size_t kMaxLds = 160 * 1024;
+// floats per row of the fp32 output tile in LDS: rows 4 apart (the two lane
+// halves) lie half the banks apart
+constexpr int kOutRow = BN + 8;
+constexpr size_t kOutBytes = (size_t)BM * kOutRow * 4;
+static_assert(kOutBytes <= kMaxLds, "output tile");
 
 // the combinations whose buffers fit one CU's LDS (all but f32 scales at
 // group size 32 with 6- or 8-bit codes)
@@ -506,11 +515,53 @@ __device__ __forceinline__ void main_loop(f32x16 (&acc)[2][2], const Ctx& t, con
     wait_vmcnt<0>();
 }
 
+// 8 columns n .. n + 7 of rows of y, through the output stage: their biases,
+// loaded once, and vector stores where rows keep 16-byte alignment
+struct RowOut {
+    void* y;
+    int N, n;
+    bool vec;
+    float bias[8];
+    __device__ __forceinline__ RowOut(void* y_, int N_, int n_, const Epilogue& ep) : y(y_), N(N_), n(n_) {
+        vec = (((uintptr_t)y) & 15) == 0 && N % (ep.out_dt == DT_F32 ? 4 : 8) == 0 && n + 8 <= N;
+#pragma unroll
+        for (int e = 0; e < 8; e++) bias[e] = ep.bias ? load_f(ep.bias, (size_t)min(n + e, N - 1), ep.bias_dt) : 0.f;
+    }
+    template <bool EPI>
+    __device__ __forceinline__ void store(int m, float (&o)[8], const Epilogue& ep) const {
+        if constexpr (EPI) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                if (ep.bias) o[e] = o[e] + bias[e];
+                o[e] = apply_act(ep.act, o[e]);
+            }
+        }
+        const size_t at = (size_t)m * N + n;
+        if (!vec) {
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (n + e < N) store_f(y, at + e, ep.out_dt, o[e]);
+        } else if (ep.out_dt == DT_F32) {
+            v4* d = reinterpret_cast<v4*>(static_cast<float*>(y) + at);
+#pragma unroll
+            for (int e = 0; e < 8; e += 4)
+                d[e / 4] = v4{__float_as_uint(o[e]), __float_as_uint(o[e + 1]), __float_as_uint(o[e + 2]),
+                              __float_as_uint(o[e + 3])};
+        } else {
+            v4 p;
+#pragma unroll
+            for (int e = 0; e < 8; e += 2)
+                p[e / 2] = ep.out_dt == DT_BF16 ? pack2<DT_BF16>(o[e], o[e + 1]) : pack2<DT_F16>(o[e], o[e + 1]);
+            *reinterpret_cast<v4*>(static_cast<uint16_t*>(y) + at) = p;
+        }
+    }
+};
+
 template <int TX, int BITS, int SB, int GS, bool EPI>
 __global__ __launch_bounds__(kThreads, 2) void qgemm_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ wq, const void* __restrict__ scales,
     const void* __restrict__ biases, void* __restrict__ y, int M, int K, int N, Epilogue ep,
-    int mtiles, int split_from, void* __restrict__ ws, uint32_t epoch) {
+    int mtiles, int split_from, int nsplit, void* __restrict__ ws, uint32_t epoch) {
     static_assert(lds_fits<BITS, GS, SB>(), "LDS budget");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -518,12 +569,21 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_kernel(
     const int wm = wave >> 1, wn = wave & 1;  // 4 x 2 waves, 64 x 64 each
     // blocks below split_from own a whole tile; the rest are the two K
     // halves (part 0: all first halves, then part 1) of tiles split_from ..
-    int tile = blockIdx.x, part = -1, KT = K / BK;
-    if (tile >= split_from) {
+    // With nsplit K parts (whole scale windows each) of all split_from tiles,
+    // block part * split_from + tile runs a part of a tile
+    int tile = blockIdx.x, part = -1, KT = K / BK, first = 0;
+    if (nsplit > 1) {
+        part = tile / split_from;
+        tile -= part * split_from;
+        const int wins = KT / 4;
+        first = wins * part / nsplit * 4;
+        KT = wins * (part + 1) / nsplit * 4 - first;
+    } else if (tile >= split_from) {
         const int r = (int)((gridDim.x - (unsigned)split_from) >> 1), i = tile - split_from;
         part = i >= r;
         tile = split_from + i - part * r;
         KT >>= 1;
+        first = part * KT;
     }
     const int mt = tile % mtiles, nt = tile / mtiles;
     const int m0 = mt * BM;
@@ -536,7 +596,7 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_kernel(
     t.wave = wave;
     t.lane = lane;
     t.KT = KT;
-    t.k0 = part > 0 ? KT : 0;
+    t.k0 = first;
     t.n0 = nt * BN;
     t.N = N;
     t.G = K / GS;
@@ -571,7 +631,7 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_kernel(
     else
         main_loop<TX, BITS, SB, GS, 1>(acc, t, scales, biases);
 
-    if (part >= 0) {
+    if (part >= 0 && nsplit == 1) {
         // A K half of a split tile: the halves meet in the workspace by the
         // protocol of qsplit.h.  The first to arrive stores its fp32 sums --
         // vector q of thread tid at byte ((slot * 16 + q) * 512 + tid) * 16
@@ -625,41 +685,101 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_kernel(
         }
     }
 
-    // ---- epilogue: 32x32 accumulator layout: lane holds column (lane % 32),
-    // VGPR v holds row 8 (v / 4) + 4 (lane / 32) + v % 4 ----
-    const int ncol = t.n0 + wn * 64 + (lane & 31);
-    const int mrow = m0 + wm * 64 + 4 * (lane >> 5);
-    if (ep.out_dt == DT_BF16 || ep.out_dt == DT_F16) {
-        uint16_t* yo = static_cast<uint16_t*>(y);
-        const bool bf = ep.out_dt == DT_BF16;
+    // ---- output: the fp32 tile through LDS (free once every wave is past its
+    // K loop; 32x32 accumulator layout: lane holds column (lane % 32), VGPR v
+    // row 8 (v / 4) + 4 (lane / 32) + v % 4), then whole 16-byte chunks of
+    // rows.  The loop stays rolled: unrolled, the activations' code (64 copies
+    // of erf or exp per thread) ran from cold instruction cache misses and
+    // took 20 us at M = 509, N = 4096 with GELU ----
+    __syncthreads();
+    float* tile_out = reinterpret_cast<float*>(lds);
+    {
+        float* d = tile_out + (wm * 64 + 4 * (lane >> 5)) * kOutRow + wn * 64 + (lane & 31);
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const int n = ncol + j * 32;
+            for (int j = 0; j < 2; j++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const int m = mrow + i * 32 + 8 * (v >> 2) + (v & 3);
-                    if (m < M && n < N) {
-                        const float o = EPI ? apply_epilogue(ep, n, acc[i][j][v]) : acc[i][j][v];
-                        yo[(size_t)m * N + n] = bf ? f32_to_bf16(o) : f32_to_f16(o);
-                    }
-                }
-            }
-    } else {
-        float* yo = static_cast<float*>(y);
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const int n = ncol + j * 32;
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const int m = mrow + i * 32 + 8 * (v >> 2) + (v & 3);
-                    if (m < M && n < N) yo[(size_t)m * N + n] = EPI ? apply_epilogue(ep, n, acc[i][j][v]) : acc[i][j][v];
-                }
-            }
+                for (int v = 0; v < 16; v++) d[(i * 32 + 8 * (v >> 2) + (v & 3)) * kOutRow + j * 32] = acc[i][j][v];
     }
+    __syncthreads();
+    // thread: columns 8 (tid % 16) ..+8 of rows tid / 16, + 32, ...
+    const int nl = tid % (BN / 8) * 8, n = t.n0 + nl;
+    if (nsplit > 1) {
+        // a K part: its tile of sums, row by row, for parts_kernel
+        float* d = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + split::kPartOffset) +
+                   (size_t)(tile * nsplit + part) * (BM * BN);
+#pragma unroll 4
+        for (int r = tid / (BN / 8); r < BM; r += kThreads / (BN / 8)) {
+            if (m0 + r >= M) break;
+#pragma unroll
+            for (int e = 0; e < 8; e += 4)
+                *reinterpret_cast<v4*>(d + r * BN + nl + e) =
+                    *reinterpret_cast<const v4*>(tile_out + r * kOutRow + nl + e);
+        }
+        return;
+    }
+    if (n >= N) return;
+    const RowOut out(y, N, n, ep);
+#pragma unroll 1
+    for (int r = tid / (BN / 8); r < BM && m0 + r < M; r += kThreads / (BN / 8)) {
+        float o[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[e] = tile_out[r * kOutRow + nl + e];
+        out.store<EPI>(m0 + r, o, ep);
+    }
+}
+
+// Sum of the K parts: 8 columns of a row per thread, the parts' tiles in part
+// order, then the output stage.  (As the last part's own work at M = 509, K =
+// 11008, N = 4096, 6-bit, 64 CUs each read 512 KiB and ran every GELU: 84 us
+// in all.  As a launch of its own over all the CUs, bound by the partials' 32
+// MiB: 69.)
+template <bool EPI>
+__global__ __launch_bounds__(256) void parts_kernel(const void* __restrict__ ws, void* __restrict__ y, int M, int N,
+                                                    Epilogue ep, int mtiles, int nsplit) {
+    const int chunks = (N + 7) / 8;
+    const unsigned id = blockIdx.x * 256u + threadIdx.x;
+    const int m = (int)(id / (unsigned)chunks), n = (int)(id % (unsigned)chunks) * 8;
+    if (m >= M) return;
+    const int tile = n / BN * mtiles + m / BM;
+    const float* p = reinterpret_cast<const float*>(static_cast<const uint8_t*>(ws) + split::kPartOffset) +
+                     (size_t)tile * nsplit * (BM * BN) + (m % BM) * BN + n % BN;
+    const RowOut out(y, N, n, ep);
+    float o[8] = {};
+#pragma unroll 4
+    for (int i = 0; i < nsplit; i++) {
+        const v4 a = *reinterpret_cast<const v4*>(p + (size_t)i * (BM * BN));
+        const v4 b = *reinterpret_cast<const v4*>(p + (size_t)i * (BM * BN) + 4);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            o[e] += __uint_as_float(a[e]);
+            o[4 + e] += __uint_as_float(b[e]);
+        }
+    }
+    out.store<EPI>(m, o, ep);
+}
+
+// K parts for a shape with few tiles (1: none, whole tiles or halves of a
+// split round), the cheapest in twentieths of a us: a step costs 1 us, a
+// part's 128 KiB 0.05 us (stored and loaded by all CUs together), the second
+// launch 3, the meeting of two halves 5.  Same box, us per launch, halves or
+// whole tiles / K parts: M = 509, K = 11008, N = 4096, 6-bit, GELU (64 tiles, 4
+// parts) 173 / 69; M = 512, K = N = 4096, 6-bit (64, 4) 41.4 / 35.6; M = 128, K
+// = N = 4096, 3-bit (32, 8) 38.7 / 24.8; N = 10000 (79, 3) 40.6 / 34.6; M = 100, K = 14336, N = 1000, 3-bit (8,
+// 32) 107 / 22; M = 70, K = 1024, N = 128, 3-bit (1, 4) 15.4 / 10.6; not taken:
+// M = 1024, K = N = 4096, 3-bit (128, 2) 48.9 / 53.7; M = 250, K = 1024, N =
+// 9000, 5-bit (71, 3) 21.8 / 26.2.
+inline int k_parts(int tiles, int KT, const QmmArgs& a) {
+    if (a.ws == nullptr || 2 * tiles > kCUs) return 1;
+    const int cap = std::min(std::min(kCUs / tiles, KT / 4),
+                             (int)((a.ws_bytes - split::kPartOffset) / ((size_t)tiles * kSplitSlotBytes)));
+    int best = 1, least = KT % 8 == 0 && a.epoch != 0u ? 10 * KT + 100 : 20 * KT;
+    for (int S = 2; S <= cap; S++) {
+        const int cost = (20 * KT + S - 1) / S + 60 + tiles * S;
+        if (cost < least) { least = cost; best = S; }
+    }
+    return best;
 }
 
 template <int TX, int BITS, int SB, int GS, bool EPI>
@@ -669,23 +789,29 @@ LuxStatus launch4_e(const QmmArgs& a, hipStream_t st) {
     } else {
         if (planned(a, "qgemm_kernel")) return LuxStatus::Ok;
         auto kern = qgemm_kernel<TX, BITS, SB, GS, EPI>;
-        constexpr size_t lds = lds_bytes<BITS, GS, SB>();
+        constexpr size_t lds = lds_bytes<BITS, GS, SB>() > kOutBytes ? lds_bytes<BITS, GS, SB>() : kOutBytes;
         static const hipError_t attr = hipFuncSetAttribute(
             reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (attr != hipSuccess) return LuxStatus::Internal;
         const int mtiles = (a.M + BM - 1) / BM, ntiles = (a.N + BN - 1) / BN;
         const int tiles = mtiles * ntiles;
+        const int nsplit = k_parts(tiles, a.K / BK, a);
         // the last round's tiles in two K halves where that round is at most
         // half full (each half a whole number of 4-step scale windows)
         const int r = tiles % kCUs;
         const int split_from =
-            r > 0 && 2 * r <= kCUs && (a.K / BK) % 8 == 0 && a.ws != nullptr && a.epoch != 0u &&
+            nsplit == 1 && r > 0 && 2 * r <= kCUs && (a.K / BK) % 8 == 0 && a.ws != nullptr && a.epoch != 0u &&
                     a.ws_bytes >= split::kPartOffset + (size_t)r * kSplitSlotBytes
                 ? tiles - r
                 : tiles;
-        hipLaunchKernelGGL(kern, dim3(tiles + (tiles - split_from)), dim3(kThreads), lds, st,
-                           static_cast<const uint16_t*>(a.x), a.wq, a.scales, a.biases, a.y, a.M, a.K,
-                           a.N, a.epi(), mtiles, split_from, a.ws, a.epoch);
+        hipLaunchKernelGGL(kern, dim3(nsplit > 1 ? tiles * nsplit : tiles + (tiles - split_from)), dim3(kThreads), lds,
+                           st, static_cast<const uint16_t*>(a.x), a.wq, a.scales, a.biases, a.y, a.M, a.K,
+                           a.N, a.epi(), mtiles, split_from, nsplit, a.ws, a.epoch);
+        if (nsplit > 1) {
+            const size_t threads = (size_t)a.M * ((a.N + 7) / 8);
+            hipLaunchKernelGGL(parts_kernel<EPI>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, a.ws, a.y,
+                               a.M, a.N, a.epi(), mtiles, nsplit);
+        }
         return hipGetLastError() == hipSuccess ? LuxStatus::Ok : LuxStatus::Internal;
     }
 }

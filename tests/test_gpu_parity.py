@@ -1094,6 +1094,47 @@ def test_group_gemm(ctx, oracle, bits, M, K, N, gs, sb, xd):
     assert np.all(np.abs(y - want) <= (32 + K / 32 + 8) * 2.0**-24 * mag)
 
 
+@pytest.mark.parametrize("bits", [2, 3, 4, 5, 6])
+@pytest.mark.parametrize("M,K,N,gs,xd,sbd,od,act", [
+    (70, 1536, 130, 64, F16, F16, F16, 3),     # 2 tiles, 6 parts of one window each, GELU
+    (257, 2816, 1003, 32, BF16, F16, BF16, 0),  # 16 tiles, 11 windows in uneven parts, odd N
+    (100, 768, 4096, 128, F16, BF16, F32, 2),  # 32 tiles, 3 parts, SiLU
+    (300, 11008, 4096, 64, BF16, BF16, F32, 0)])  # 64 tiles, 43 windows in 4 parts
+def test_lds_gemm_k_parts(ctx, oracle, bits, M, K, N, gs, xd, sbd, od, act):
+    """The LDS-dequant GEMM in K parts summed by a second launch, with the
+    fused output stage there, twice (the same bits), against the
+    dequantize-to-T form."""
+    from mlx_amd import runtime
+    O = oracle
+    assert ctx.kernel_name(M, K, N, gs, bits, xd, sbd, od) == "qgemm_kernel"
+    x, w_q, s, b, _ = O.make_problem(M, K, N, bits, gs, xd, sbd, seed=8300 + M + bits)
+    rows = np.unique(np.r_[0, M // 3, M - 1])
+    xs = np.ascontiguousarray(x[rows])
+    acc = O.quantized_matmul(xs, w_q, s, b, len(rows), K, N, gs, bits, xd, sbd, F32, variant="omp", w_round=xd)
+    bias = O.rng_normal(N, seed=8400 + N).astype(np.float32)
+    bufs = [ctx.upload(a) for a in (x, w_q, s, b)]
+    bb = ctx.upload(bias)
+    out = ctx.alloc(M * N * runtime.esize(od))
+    try:
+        ys = []
+        for _ in range(2):
+            print(f"[case] K parts M={M} K={K} N={N} b{bits} act={act}", flush=True)
+            ctx.quantized_matmul_fused(*bufs, bb if act else None, out, M, K, N, gs, bits, xd, sbd, F32, od, act)
+            ys.append(out.download(runtime.np_dtype(od), (M, N)))
+    finally:
+        for t in bufs + [bb, out]:
+            t.free()
+    assert np.array_equal(ys[0], ys[1])
+    want = acc.astype(np.float64)
+    if act:
+        want = want + bias
+        from math import erf
+        want = want / (1 + np.exp(-want)) if act == 2 else \
+            0.5 * want * (1 + np.vectorize(erf)(want / np.sqrt(2.0)))
+    check_output(O, np.ascontiguousarray(ys[0][rows]), O.from_f32(want.astype(np.float32), od), od,
+                 f"K parts b{bits} M{M} K{K} N{N}")
+
+
 def test_f32_gemm_special_values(ctx, oracle):
     """An infinity or a NaN in a row of x reaches that row's outputs and no
     other, and x of 2^120, all mantissa bits set, stays finite in its three
