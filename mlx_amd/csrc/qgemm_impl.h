@@ -45,14 +45,15 @@
 // every part stores its fp32 tile, and a second launch adds them in part
 // order and stores y.
 #pragma once
-#include <algorithm>
-
 #include "kernels.h"
 #include "qcommon.h"
 #include "qsplit.h"
+#include "qtile_out.h"
 
 namespace lxq {
 namespace gemm {
+
+using namespace tileout;
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -69,7 +70,6 @@ constexpr int kXStages = 3;
 constexpr int kWStageBytes = BN * BK * 2;  // 16384
 // tail split: CUs of the target (MI355X: 256); the workspace layout and the
 // protocol of the split tiles are qsplit.h's
-constexpr int kCUs = 256;
 constexpr uint32_t kSplitSlotBytes = BM * BN * 4;  // one K half of one tile, fp32
 static_assert(split::kPartOffset + (size_t)kCUs / 2 * kSplitSlotBytes <= kSplitWorkspaceBytes, "workspace size");
 static_assert(kCUs / 2 <= split::kMaxHalfTiles, "split tiles within the workspace's counter words");
@@ -515,48 +515,6 @@ __device__ __forceinline__ void main_loop(f32x16 (&acc)[2][2], const Ctx& t, con
     wait_vmcnt<0>();
 }
 
-// 8 columns n .. n + 7 of rows of y, through the output stage: their biases,
-// loaded once, and vector stores where rows keep 16-byte alignment
-struct RowOut {
-    void* y;
-    int N, n;
-    bool vec;
-    float bias[8];
-    __device__ __forceinline__ RowOut(void* y_, int N_, int n_, const Epilogue& ep) : y(y_), N(N_), n(n_) {
-        vec = (((uintptr_t)y) & 15) == 0 && N % (ep.out_dt == DT_F32 ? 4 : 8) == 0 && n + 8 <= N;
-#pragma unroll
-        for (int e = 0; e < 8; e++) bias[e] = ep.bias ? load_f(ep.bias, (size_t)min(n + e, N - 1), ep.bias_dt) : 0.f;
-    }
-    template <bool EPI>
-    __device__ __forceinline__ void store(int m, float (&o)[8], const Epilogue& ep) const {
-        if constexpr (EPI) {
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                if (ep.bias) o[e] = o[e] + bias[e];
-                o[e] = apply_act(ep.act, o[e]);
-            }
-        }
-        const size_t at = (size_t)m * N + n;
-        if (!vec) {
-#pragma unroll
-            for (int e = 0; e < 8; e++)
-                if (n + e < N) store_f(y, at + e, ep.out_dt, o[e]);
-        } else if (ep.out_dt == DT_F32) {
-            v4* d = reinterpret_cast<v4*>(static_cast<float*>(y) + at);
-#pragma unroll
-            for (int e = 0; e < 8; e += 4)
-                d[e / 4] = v4{__float_as_uint(o[e]), __float_as_uint(o[e + 1]), __float_as_uint(o[e + 2]),
-                              __float_as_uint(o[e + 3])};
-        } else {
-            v4 p;
-#pragma unroll
-            for (int e = 0; e < 8; e += 2)
-                p[e / 2] = ep.out_dt == DT_BF16 ? pack2<DT_BF16>(o[e], o[e + 1]) : pack2<DT_F16>(o[e], o[e + 1]);
-            *reinterpret_cast<v4*>(static_cast<uint16_t*>(y) + at) = p;
-        }
-    }
-};
-
 template <int TX, int BITS, int SB, int GS, bool EPI>
 __global__ __launch_bounds__(kThreads, 2) void qgemm_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ wq, const void* __restrict__ scales,
@@ -730,58 +688,6 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_kernel(
     }
 }
 
-// Sum of the K parts: 8 columns of a row per thread, the parts' tiles in part
-// order, then the output stage.  (As the last part's own work at M = 509, K =
-// 11008, N = 4096, 6-bit, 64 CUs each read 512 KiB and ran every GELU: 84 us
-// in all.  As a launch of its own over all the CUs, bound by the partials' 32
-// MiB: 69.)
-template <bool EPI>
-__global__ __launch_bounds__(256) void parts_kernel(const void* __restrict__ ws, void* __restrict__ y, int M, int N,
-                                                    Epilogue ep, int mtiles, int nsplit) {
-    const int chunks = (N + 7) / 8;
-    const unsigned id = blockIdx.x * 256u + threadIdx.x;
-    const int m = (int)(id / (unsigned)chunks), n = (int)(id % (unsigned)chunks) * 8;
-    if (m >= M) return;
-    const int tile = n / BN * mtiles + m / BM;
-    const float* p = reinterpret_cast<const float*>(static_cast<const uint8_t*>(ws) + split::kPartOffset) +
-                     (size_t)tile * nsplit * (BM * BN) + (m % BM) * BN + n % BN;
-    const RowOut out(y, N, n, ep);
-    float o[8] = {};
-#pragma unroll 4
-    for (int i = 0; i < nsplit; i++) {
-        const v4 a = *reinterpret_cast<const v4*>(p + (size_t)i * (BM * BN));
-        const v4 b = *reinterpret_cast<const v4*>(p + (size_t)i * (BM * BN) + 4);
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            o[e] += __uint_as_float(a[e]);
-            o[4 + e] += __uint_as_float(b[e]);
-        }
-    }
-    out.store<EPI>(m, o, ep);
-}
-
-// K parts for a shape with few tiles (1: none, whole tiles or halves of a
-// split round), the cheapest in twentieths of a us: a step costs 1 us, a
-// part's 128 KiB 0.05 us (stored and loaded by all CUs together), the second
-// launch 3, the meeting of two halves 5.  Same box, us per launch, halves or
-// whole tiles / K parts: M = 509, K = 11008, N = 4096, 6-bit, GELU (64 tiles, 4
-// parts) 173 / 69; M = 512, K = N = 4096, 6-bit (64, 4) 41.4 / 35.6; M = 128, K
-// = N = 4096, 3-bit (32, 8) 38.7 / 24.8; N = 10000 (79, 3) 40.6 / 34.6; M = 100, K = 14336, N = 1000, 3-bit (8,
-// 32) 107 / 22; M = 70, K = 1024, N = 128, 3-bit (1, 4) 15.4 / 10.6; not taken:
-// M = 1024, K = N = 4096, 3-bit (128, 2) 48.9 / 53.7; M = 250, K = 1024, N =
-// 9000, 5-bit (71, 3) 21.8 / 26.2.
-inline int k_parts(int tiles, int KT, const QmmArgs& a) {
-    if (a.ws == nullptr || 2 * tiles > kCUs) return 1;
-    const int cap = std::min(std::min(kCUs / tiles, KT / 4),
-                             (int)((a.ws_bytes - split::kPartOffset) / ((size_t)tiles * kSplitSlotBytes)));
-    int best = 1, least = KT % 8 == 0 && a.epoch != 0u ? 10 * KT + 100 : 20 * KT;
-    for (int S = 2; S <= cap; S++) {
-        const int cost = (20 * KT + S - 1) / S + 60 + tiles * S;
-        if (cost < least) { least = cost; best = S; }
-    }
-    return best;
-}
-
 template <int TX, int BITS, int SB, int GS, bool EPI>
 LuxStatus launch4_e(const QmmArgs& a, hipStream_t st) {
     if constexpr (!lds_fits<BITS, GS, SB>()) {
@@ -795,7 +701,9 @@ LuxStatus launch4_e(const QmmArgs& a, hipStream_t st) {
         if (attr != hipSuccess) return LuxStatus::Internal;
         const int mtiles = (a.M + BM - 1) / BM, ntiles = (a.N + BN - 1) / BN;
         const int tiles = mtiles * ntiles;
-        const int nsplit = k_parts(tiles, a.K / BK, a);
+        // (scale windows of 4 steps; halves of whole windows)
+        const int KT = a.K / BK;
+        const int nsplit = k_parts(tiles, KT, KT / 4, KT % 8 == 0, 20, a);
         // the last round's tiles in two K halves where that round is at most
         // half full (each half a whole number of 4-step scale windows)
         const int r = tiles % kCUs;
@@ -807,11 +715,7 @@ LuxStatus launch4_e(const QmmArgs& a, hipStream_t st) {
         hipLaunchKernelGGL(kern, dim3(nsplit > 1 ? tiles * nsplit : tiles + (tiles - split_from)), dim3(kThreads), lds,
                            st, static_cast<const uint16_t*>(a.x), a.wq, a.scales, a.biases, a.y, a.M, a.K,
                            a.N, a.epi(), mtiles, split_from, nsplit, a.ws, a.epoch);
-        if (nsplit > 1) {
-            const size_t threads = (size_t)a.M * ((a.N + 7) / 8);
-            hipLaunchKernelGGL(parts_kernel<EPI>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, a.ws, a.y,
-                               a.M, a.N, a.epi(), mtiles, nsplit);
-        }
+        if (nsplit > 1) launch_parts<BM, BN, EPI>(a, mtiles, nsplit, st);
         return hipGetLastError() == hipSuccess ? LuxStatus::Ok : LuxStatus::Internal;
     }
 }

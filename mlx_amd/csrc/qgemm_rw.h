@@ -43,9 +43,10 @@
 // product is exactly s q: each value is fmaf(s, q, b) bit for bit, one
 // instruction per code (2^(24-p) s is exact for |s| < 2^103).
 //
-// Work units: tiles (K halves for a split last round, K parts for a shape
-// with few tiles; qsplit.h).  Grid: one block per unit, or, where there are
-// more units than CUs and the output is 16-bit, one block per CU running
+// Work units: tiles (K halves for a split last round, qsplit.h; K parts for a
+// shape with few tiles, summed by a second launch, qtile_out.h).  Grid: one
+// block per unit, or, where there are more units than CUs, the output is
+// 16-bit and no output stage is fused, one block per CU running
 // units b, b + 256, ... (whole tiles first, halves last): at each hand-over
 // the next unit's first transfers go out before the finished tile is
 // staged and stored, so its prologue latency runs under the output stage,
@@ -54,11 +55,10 @@
 // (block b runs on XCD b % 8) in 4 x 8 groups of M x N tiles, so the 32
 // blocks an XCD runs at once share 4 x slabs and 8 W slabs in its L2.
 #pragma once
-#include <cstdlib>
-
 #include "kernels.h"
 #include "qcommon.h"
 #include "qsplit.h"
+#include "qtile_out.h"
 
 namespace lxq {
 namespace rw {
@@ -70,7 +70,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 
 constexpr int BN = 256, BK = 64;
-constexpr int kCUs = 256;
+using tileout::kCUs;
 
 template <int TX_, int BITS_, int SB_, int GS_, int NW_, int D_, int BAR_, int MT_>
 struct Cfg {
@@ -441,11 +441,13 @@ __device__ __forceinline__ Unit unit_of(int u, int tiles, int split_from, int ns
     w.k0 = 0;
     if (nsplit > 1) {
         // K parts: unit u = part * tiles + tile (the blocks running together
-        // share a K range, i.e. the same x columns)
+        // share a K range, i.e. the same x columns), each a whole number of
+        // unrolled loops
         w.tile = u % tiles;
         w.part = u / tiles;
-        w.KT = KT / nsplit;
-        w.k0 = w.part * w.KT;
+        const int loops = KT / C::kUnroll;
+        w.k0 = loops * w.part / nsplit * C::kUnroll;
+        w.KT = loops * (w.part + 1) / nsplit * C::kUnroll - w.k0;
     } else if (u >= split_from) {
         // units below split_from are whole tiles; the rest are the two K
         // halves (all first halves, then all second halves) of tiles split_from ..
@@ -663,7 +665,9 @@ __global__ __launch_bounds__(C::kThreads, 1) void qgemm_rw_kernel(
         // no transfer may still be landing when LDS is next written
         wait_vm<0>();
         const int un = u + (int)gridDim.x;
-        if (un >= units || w.part >= 0) break;
+        // (with the fused output stage a block runs one unit: the stage is the
+        // rolled loop below)
+        if (EPI || un >= units || w.part >= 0) break;
 
         // ---- hand-over to unit un: every wave is past its K loop (the
         // rings are free after this barrier) ----
@@ -713,63 +717,7 @@ __global__ __launch_bounds__(C::kThreads, 1) void qgemm_rw_kernel(
     constexpr uint32_t kSlot = (uint32_t)(kVec * C::kThreads * 16);  // = BM BN 4
     const uint32_t voff = (uint32_t)tid * 16u;
     uint32_t* word = reinterpret_cast<uint32_t*>(lds);  // every transfer has landed
-    if (nsplit > 1) {
-        // ---- K parts: every part stores its sums; the last to count in adds
-        // all nsplit of them in part order (the same bits whichever part is
-        // last) and stores y; it also returns the tile's counter to zero ----
-        const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(
-            static_cast<uint8_t*>(ws) + split::kPartOffset, 0, (int)((uint32_t)(tiles * nsplit) * kSlot), 0x00020000);
-        const uint32_t slot = (uint32_t)(w.tile * nsplit + w.part) * kSlot;
-#pragma unroll
-        for (int q = 0; q < kVec; q++) {
-            const f32x16& a = acc[q / (4 * NT)][(q / 4) % NT];
-            const int v = 4 * (q % 4);
-            __builtin_amdgcn_raw_buffer_store_b128(
-                u4{__float_as_uint(a[v]), __float_as_uint(a[v + 1]), __float_as_uint(a[v + 2]), __float_as_uint(a[v + 3])},
-                pr, voff, slot + (uint32_t)q * (C::kThreads * 16u), split::kCachePolicyDevice);
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        barrier();
-        if (tid == 0) *word = split::count_part(ws, w.tile, nsplit) ? 1u : 0u;
-        barrier();
-        if (*word == 0u) return;
-        const uint32_t first = (uint32_t)(w.tile * nsplit) * kSlot;
-#pragma unroll
-        for (int q = 0; q < kVec; q++) {
-            f32x16& a = acc[q / (4 * NT)][(q / 4) % NT];
-            const int v = 4 * (q % 4);
-            a[v] = a[v + 1] = a[v + 2] = a[v + 3] = 0.f;
-        }
-        // kPB parts' sums in flight together (32 vectors per thread: one
-        // memory round trip per kPB parts, not per part); nsplit is a power
-        // of two, so whole batches or a single one
-        constexpr int kPB = kVec >= 32 ? 1 : 32 / kVec;
-        for (int p0 = 0; p0 < nsplit; p0 += kPB) {
-            u4 o[kPB][kVec];
-#pragma unroll
-            for (int pp = 0; pp < kPB; pp++)
-#pragma unroll
-                for (int q = 0; q < kVec; q++)
-                    o[pp][q] = p0 + pp < nsplit
-                                   ? __builtin_amdgcn_raw_buffer_load_b128(
-                                         pr, voff, first + (uint32_t)(p0 + pp) * kSlot + (uint32_t)q * (C::kThreads * 16u),
-                                         split::kCachePolicyDevice)
-                                   : u4{0u, 0u, 0u, 0u};
-#pragma unroll
-            for (int pp = 0; pp < kPB; pp++) {
-                if (p0 + pp >= nsplit) break;
-#pragma unroll
-                for (int q = 0; q < kVec; q++) {
-                    f32x16& a = acc[q / (4 * NT)][(q / 4) % NT];
-                    const int v = 4 * (q % 4);
-                    a[v] += __uint_as_float(o[pp][q].x);
-                    a[v + 1] += __uint_as_float(o[pp][q].y);
-                    a[v + 2] += __uint_as_float(o[pp][q].z);
-                    a[v + 3] += __uint_as_float(o[pp][q].w);
-                }
-            }
-        }
-    } else if (w.part >= 0) {
+    if (nsplit == 1 && w.part >= 0) {
         // ---- split last round: the two K halves meet (qsplit.h) ----
         const int st = w.tile - split_from;
         const uint32_t nslots = (uint32_t)(tiles - split_from);
@@ -813,59 +761,76 @@ __global__ __launch_bounds__(C::kThreads, 1) void qgemm_rw_kernel(
     // ---- output: lane holds column c of each 32 x 32 tile, VGPR v row
     // 8 (v / 4) + 4 h + v % 4.  The tile goes through LDS (free now: every
     // transfer has landed and every wave is past the K loop at the barrier)
-    // so that the stores to y are whole 16-byte chunks of rows, in one pass
-    // (two of half the rows for fp32 outputs of 128-row tiles).
+    // so that the stores are whole 16-byte chunks of rows: 16-bit values in
+    // one pass; fp32 ones (an fp32 y, a K part's sums, and with the fused
+    // output stage, which a rolled loop applies to the rows read back) in two
+    // passes of half the rows for 128-row tiles.
     const bool f32_out = ep.out_dt == DT_F32;
-    const int esz = f32_out ? 4 : 2;
-    const int rs = BN * esz + 16;  // LDS row stride: rows m and m + 4 in different banks
-    // vector stores need 16-byte aligned rows: N a multiple of 16 / esz, y aligned
-    const bool vec = (((uintptr_t)y) & 15) == 0 && (N % (16 / esz)) == 0;
-    const int passes = BM * rs > C::kLds ? 2 : 1, prow = BM / passes;
-    for (int ps = 0; ps < passes; ps++) {
+    if (!EPI && !f32_out && nsplit == 1) {
+        constexpr int rs = BN * 2 + 16;  // LDS row stride: rows m and m + 4 in different banks
+        // vector stores need 16-byte aligned rows: N a multiple of 8, y aligned
+        const bool vec = (((uintptr_t)y) & 15) == 0 && N % 8 == 0;
         barrier();
-        if (!f32_out) {
-            // one pass (prow = BM)
-            if (ep.out_dt == DT_BF16) stage16<C, EPI, DT_BF16>(lds, rs, acc, ep, n0, N, wave, c, h);
-            else stage16<C, EPI, DT_F16>(lds, rs, acc, ep, n0, N, wave, c, h);
-        } else {
-#pragma unroll
-            for (int i = 0; i < MT; i++) {
-                if (i * 32 / prow != ps) continue;
-#pragma unroll
-                for (int tt = 0; tt < NT; tt++) {
-                    const int nl = wave * C::WN + 32 * tt + c;  // column within the tile
-                    const int n = n0 + nl;
-#pragma unroll
-                    for (int v = 0; v < 16; v++) {
-                        const int ml = 32 * i + 8 * (v >> 2) + 4 * h + (v & 3) - ps * prow;
-                        float o = acc[i][tt][v];
-                        if constexpr (EPI) {
-                            if (n < N) o = apply_epilogue(ep, (size_t)n, o);
-                        }
-                        *reinterpret_cast<float*>(lds + ml * rs + nl * 4) = o;
-                    }
-                }
-            }
-        }
+        if (ep.out_dt == DT_BF16) stage16<C, EPI, DT_BF16>(lds, rs, acc, ep, n0, N, wave, c, h);
+        else stage16<C, EPI, DT_F16>(lds, rs, acc, ep, n0, N, wave, c, h);
         barrier();
-        // row r of the pass: BN * esz bytes = cpr 16-byte chunks
-        const int cpr = BN * esz / 16;
-        for (int q = tid; q < prow * cpr; q += C::kThreads) {
-            const int rl = q / cpr, ch = q % cpr;
-            const int m = m0 + ps * prow + rl, n = n0 + ch * (16 / esz);
+        // row r: BN * 2 bytes = 32 16-byte chunks
+        for (int q = tid; q < BM * 32; q += C::kThreads) {
+            const int rl = q / 32, ch = q % 32;
+            const int m = m0 + rl, n = n0 + ch * 8;
             if (m >= M || n >= N) continue;
             const u4 val = *reinterpret_cast<const u4*>(lds + rl * rs + ch * 16);
-            uint8_t* dst = static_cast<uint8_t*>(y) + ((size_t)m * N + n) * esz;
-            if (vec && n + 16 / esz <= N) {
+            uint8_t* dst = static_cast<uint8_t*>(y) + ((size_t)m * N + n) * 2;
+            if (vec && n + 8 <= N) {
                 *reinterpret_cast<u4*>(dst) = val;
-            } else if (f32_out) {
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    if (n + e < N) reinterpret_cast<uint32_t*>(dst)[e] = val[e];
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; e++)
                     if (n + e < N) reinterpret_cast<uint16_t*>(dst)[e] = (uint16_t)(val[e >> 1] >> (16 * (e & 1)));
+            }
+        }
+        return;
+    }
+    constexpr int rs = BN * 4 + 16;
+    constexpr int passes = BM * rs > C::kLds ? 2 : 1, prow = BM / passes;
+    // thread: columns 8 (tid % 32) ..+8 of rows tid / 32, + kThreads / 32, ...
+    const int nl = tid % 32 * 8, n = n0 + nl;
+    const tileout::RowOut out(y, N, n < N ? n : N - 1, ep);
+    float* part = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + split::kPartOffset) +
+                  (size_t)(w.tile * nsplit + (nsplit > 1 ? w.part : 0)) * (BM * BN) + nl;
+#pragma unroll
+    for (int ps = 0; ps < passes; ps++) {
+        barrier();
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            if (i * 32 / prow != ps) continue;
+#pragma unroll
+            for (int tt = 0; tt < NT; tt++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    const int ml = 32 * i + 8 * (v >> 2) + 4 * h + (v & 3) - ps * prow;
+                    *reinterpret_cast<float*>(lds + ml * rs + (wave * C::WN + 32 * tt + c) * 4) = acc[i][tt][v];
+                }
+        }
+        barrier();
+#pragma unroll 1
+        for (int rl = tid / 32; rl < prow; rl += C::kThreads / 32) {
+            const int r = ps * prow + rl, m = m0 + r;
+            if (m >= M || n >= N) break;
+            const u4* src = reinterpret_cast<const u4*>(lds + rl * rs + nl * 4);
+            const u4 a = src[0], b = src[1];
+            if (nsplit > 1) {
+                u4* d = reinterpret_cast<u4*>(part + (size_t)r * BN);
+                d[0] = a;
+                d[1] = b;
+            } else {
+                float o[8];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    o[e] = __uint_as_float(a[e]);
+                    o[4 + e] = __uint_as_float(b[e]);
+                }
+                out.store<EPI>(m, o, ep);
             }
         }
     }
@@ -879,20 +844,6 @@ inline bool applies(int M, int K, int N, int bits, int x_dtype) {
            N > 0 && (size_t)M * K * 2 < (1ull << 32) && (size_t)N * K * bits / 8 < (1ull << 32);
 }
 
-// K parts for a shape with few tiles: the largest power of two (at most 16)
-// that keeps the grid within one block per CU, every part a whole number of
-// unrolled loops, and the parts' sums within the workspace; 1 for shapes
-// with at least half a round of tiles (their last round splits instead)
-template <class C>
-inline int k_parts(int tiles, int KT, const QmmArgs& a) {
-    if (a.ws == nullptr || 2 * tiles > kCUs || tiles > split::kMaxPartTiles) return 1;
-    int S = 1;
-    while (S < 16 && tiles * 2 * S <= kCUs && KT % (2 * S * C::kUnroll) == 0 &&
-           split::kPartOffset + (size_t)tiles * 2 * S * C::BM * BN * 4 <= a.ws_bytes)
-        S *= 2;
-    return S;
-}
-
 template <class C, bool EPI>
 LuxStatus launch_e(const QmmArgs& a, hipStream_t st) {
     if (planned(a, "qgemm_rw_kernel")) return LuxStatus::Ok;
@@ -903,7 +854,8 @@ LuxStatus launch_e(const QmmArgs& a, hipStream_t st) {
     if (attr != hipSuccess) return LuxStatus::Internal;
     const int mtiles = (a.M + C::BM - 1) / C::BM, ntiles = (a.N + BN - 1) / BN;
     const int tiles = mtiles * ntiles, KT = a.K / BK;
-    const int nsplit = k_parts<C>(tiles, KT, a);
+    // K parts of whole unrolled loops each; a step of the tile costs 0.9 us
+    const int nsplit = tileout::k_parts(tiles, KT, KT / C::kUnroll, (KT / 2) % C::kUnroll == 0, 18, a);
     // with whole tiles: the last round's tiles in two K halves where that
     // round is at most half full (each half a whole number of unrolled loops)
     const int r = tiles % kCUs;
@@ -915,14 +867,19 @@ LuxStatus launch_e(const QmmArgs& a, hipStream_t st) {
     const int units = nsplit > 1 ? tiles * nsplit : tiles + (tiles - split_from);
     // one block per CU where there are more units than CUs and the
     // hand-over's stores apply: 16-bit output in whole 16-byte chunks at
-    // 31-bit offsets (chunks past the end are dropped by offset)
-    const bool persist = nsplit == 1 && units > kCUs && a.out_dtype != DT_F32 && (((uintptr_t)a.y) & 15) == 0 &&
+    // 31-bit offsets (chunks past the end are dropped by offset).  Not with
+    // the fused output stage: unrolled in the hand-over its 64 activations per
+    // thread ran from cold instruction cache lines (M = 2048, K = 4096, N =
+    // 14336, 4-bit: GELU 285 us, SiLU 278, against 272 and 262 in the rolled
+    // loop of one block per unit; 224 without)
+    const bool persist = !EPI && nsplit == 1 && units > kCUs && a.out_dtype != DT_F32 && (((uintptr_t)a.y) & 15) == 0 &&
                          a.N % 8 == 0 && (size_t)a.M * a.N * 2 < 0x80000000ull;
     const int blocks = persist ? kCUs : units;
     const int lds = persist ? kLdsMax : C::kLds;
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(C::kThreads), lds, st, static_cast<const uint16_t*>(a.x), a.wq,
                        a.scales, a.biases, a.y, a.M, a.K, a.N, a.epi(), mtiles, ntiles, split_from, nsplit, a.ws,
                        a.epoch, units);
+    if (nsplit > 1) tileout::launch_parts<C::BM, BN, EPI>(a, mtiles, nsplit, st);
     return hipGetLastError() == hipSuccess ? LuxStatus::Ok : LuxStatus::Internal;
 }
 

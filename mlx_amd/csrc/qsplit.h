@@ -8,9 +8,8 @@
 //                        kernel returns each to zero at the end of a launch)
 //   bytes [1024, 1536)   large-GEMM split-tile arrival counters (128 words)
 //   bytes [1536, 2048)   large-GEMM split-tile flags (128 words)
-//   bytes [2048, 3072)   K-part counters of the large and the group-wise
-//                        GEMMs (256 words; the last part of a tile returns
-//                        its counter to zero)
+//   bytes [2048, 3072)   group-wise GEMM K-part counters (256 words; the last
+//                        part of a tile returns its counter to zero)
 //   bytes [4096, ...)    partial sums of whichever kernel runs (meaningful
 //                        only within the launch that writes them)
 // The two kernels' words never overlap, so neither can disturb the other's
@@ -53,7 +52,8 @@ static_assert(kHalfFlagWord + kMaxHalfTiles <= kPartCounterWord &&
                   (size_t)(kPartCounterWord + kMaxPartTiles) * 4 <= kPartOffset,
               "K-part counters between the flags and the partial sums");
 
-// K parts (register-W, LDS-dequant and group-wise GEMMs): one thread per block, after the block's sums
+// K parts (group-wise GEMM; the large GEMMs' are summed by a second launch,
+// qtile_out.h): one thread per block, after the block's sums
 // are stored (vmcnt(0)) and the block has met at a barrier.  true for the
 // last of the tile's `parts` to count in, which also sets the counter back
 // to zero for the next launch (every other part has counted in by then).

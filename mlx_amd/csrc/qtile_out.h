@@ -1,0 +1,135 @@
+// qtile_out.h -- what the large GEMMs share past their K loops: rows of y
+// through the output stage, and K parts: their number, and the launch that
+// adds them.
+#pragma once
+#include <algorithm>
+
+#include "kernels.h"
+#include "qcommon.h"
+#include "qsplit.h"
+
+namespace lxq {
+namespace tileout {
+
+typedef uint32_t t4 __attribute__((ext_vector_type(4), aligned(16)));
+constexpr int kCUs = 256;
+constexpr size_t kTileBytes = 128 * 1024;  // both GEMMs' tiles hold 32 Ki fp32 sums
+
+// two fp32 values -> a packed pair of T, RNE
+template <int T>
+__device__ __forceinline__ uint32_t pair(float a, float b) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    if constexpr (T == DT_BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, b2));
+    else return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, h2));
+}
+
+// 8 columns n .. n + 7 of rows of y, through the output stage: their biases,
+// loaded once, and vector stores where rows keep 16-byte alignment
+struct RowOut {
+    void* y;
+    int N, n;
+    bool vec;
+    float bias[8];
+    __device__ __forceinline__ RowOut(void* y_, int N_, int n_, const Epilogue& ep) : y(y_), N(N_), n(n_) {
+        vec = (((uintptr_t)y) & 15) == 0 && N % (ep.out_dt == DT_F32 ? 4 : 8) == 0 && n + 8 <= N;
+#pragma unroll
+        for (int e = 0; e < 8; e++) bias[e] = ep.bias ? load_f(ep.bias, (size_t)min(n + e, N - 1), ep.bias_dt) : 0.f;
+    }
+    template <bool EPI>
+    __device__ __forceinline__ void store(int m, float (&o)[8], const Epilogue& ep) const {
+        if constexpr (EPI) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                if (ep.bias) o[e] = o[e] + bias[e];
+                o[e] = apply_act(ep.act, o[e]);
+            }
+        }
+        const size_t at = (size_t)m * N + n;
+        if (!vec) {
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (n + e < N) store_f(y, at + e, ep.out_dt, o[e]);
+        } else if (ep.out_dt == DT_F32) {
+            t4* d = reinterpret_cast<t4*>(static_cast<float*>(y) + at);
+#pragma unroll
+            for (int e = 0; e < 8; e += 4)
+                d[e / 4] = t4{__float_as_uint(o[e]), __float_as_uint(o[e + 1]), __float_as_uint(o[e + 2]),
+                              __float_as_uint(o[e + 3])};
+        } else {
+            t4 p;
+#pragma unroll
+            for (int e = 0; e < 8; e += 2)
+                p[e / 2] = ep.out_dt == DT_BF16 ? pair<DT_BF16>(o[e], o[e + 1]) : pair<DT_F16>(o[e], o[e + 1]);
+            *reinterpret_cast<t4*>(static_cast<uint16_t*>(y) + at) = p;
+        }
+    }
+};
+
+// Sum of the K parts: 8 columns of a row per thread, the parts' tiles in part
+// order, then the output stage.  (As the last part's own work at M = 509, K =
+// 11008, N = 4096, 6-bit, 64 CUs each read 512 KiB and ran every GELU: 84 us
+// in all.  As a launch of its own over all the CUs, bound by the partials' 32
+// MiB: 69.)
+template <int BM, int BN, bool EPI>
+__global__ __launch_bounds__(256) void parts_kernel(const void* __restrict__ ws, void* __restrict__ y, int M, int N,
+                                                    Epilogue ep, int mtiles, int nsplit) {
+    const int chunks = (N + 7) / 8;
+    const unsigned id = blockIdx.x * 256u + threadIdx.x;
+    const int m = (int)(id / (unsigned)chunks), n = (int)(id % (unsigned)chunks) * 8;
+    if (m >= M) return;
+    const int tile = n / BN * mtiles + m / BM;
+    const float* p = reinterpret_cast<const float*>(static_cast<const uint8_t*>(ws) + split::kPartOffset) +
+                     (size_t)tile * nsplit * (BM * BN) + (m % BM) * BN + n % BN;
+    const RowOut out(y, N, n, ep);
+    float o[8] = {};
+#pragma unroll 4
+    for (int i = 0; i < nsplit; i++) {
+        const t4 a = *reinterpret_cast<const t4*>(p + (size_t)i * (BM * BN));
+        const t4 b = *reinterpret_cast<const t4*>(p + (size_t)i * (BM * BN) + 4);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            o[e] += __uint_as_float(a[e]);
+            o[4 + e] += __uint_as_float(b[e]);
+        }
+    }
+    out.store<EPI>(m, o, ep);
+}
+
+template <int BM, int BN, bool EPI>
+void launch_parts(const QmmArgs& a, int mtiles, int nsplit, hipStream_t st) {
+    static_assert((size_t)BM * BN * 4 == kTileBytes, "tile of sums");
+    const size_t threads = (size_t)a.M * ((a.N + 7) / 8);
+    hipLaunchKernelGGL((parts_kernel<BM, BN, EPI>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, a.ws,
+                       a.y, a.M, a.N, a.epi(), mtiles, nsplit);
+}
+
+// K parts for a shape with few tiles (1: none, whole tiles or halves of a
+// split round) of KT steps, at most `most`, the cheapest in twentieths of a
+// us: a step costs `step` (LDS-dequant GEMM: 20), a part's 128 KiB 1 (stored
+// and loaded by all CUs together), the second launch 60, the meeting of two
+// halves 100.  Same box, us per launch, halves or whole tiles / K parts
+// (tiles, parts): LDS-dequant GEMM M = 509, K = 11008, N = 4096, 6-bit, GELU
+// (64, 4) 173 / 69; M = 512, K = N = 4096, 6-bit (64, 4) 41.4 / 35.6; M = 128,
+// K = N = 4096, 3-bit (32, 8) 38.7 / 24.8, N = 10000 (79, 3) 40.6 / 34.6; M =
+// 100, K = 14336, N = 1000, 3-bit (8, 32) 107 / 22; M = 70, K = 1024, N = 128,
+// 3-bit (1, 4) 15.4 / 10.6; not taken: M = 1024, K = N = 4096, 3-bit (128, 2)
+// 48.9 / 53.7; M = 250, K = 1024, N = 9000, 5-bit (71, 3) 21.8 / 26.2.
+// Register-W GEMM, its parts summed by the last to arrive / by the launch:
+// 8-bit M = 100, K = 14336, N = 1000 55.2 / 20.8; 4-bit M = 128, K = 14336, N =
+// 4096 49.5 / 31.2; M = 80, K = 4096, N = 1000 24.1 / 14.5.
+inline int k_parts(int tiles, int KT, int most, bool halves, int step, const QmmArgs& a) {
+    if (a.ws == nullptr || 2 * tiles > kCUs) return 1;
+    const int cap = std::min(std::min(kCUs / tiles, most),
+                             (int)((a.ws_bytes - split::kPartOffset) / ((size_t)tiles * kTileBytes)));
+    int best = 1, least = halves && a.epoch != 0u ? step * KT / 2 + 100 : step * KT;
+    for (int S = 2; S <= cap; S++) {
+        const int cost = (step * KT + S - 1) / S + 60 + tiles * S;
+        if (cost < least) { least = cost; best = S; }
+    }
+    return best;
+}
+
+}  // namespace tileout
+}  // namespace lxq
