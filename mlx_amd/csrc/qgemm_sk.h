@@ -136,9 +136,9 @@ __global__ __launch_bounds__(64 * kWaves, 2) void qgemm_sk_kernel(
     const int j = lane & 31, h = lane >> 5;
     const int tile = blockIdx.x / S, part = blockIdx.x % S;
     const int n0 = tile * kCols;
-    const int Kp = K / S;                    // a multiple of kSS
-    const int k0 = part * Kp;
-    const int nss = Kp / kSS;
+    const int all = K / kSS, ss0 = all * part / S;  // the part's super-steps
+    const int k0 = ss0 * kSS;
+    const int nss = all * (part + 1) / S - ss0;
     const uint32_t row_bytes = (uint32_t)K * BITS / 8;
     const int G = K / GS;
     constexpr int kSb = SB == DT_F32 ? 4 : 2;

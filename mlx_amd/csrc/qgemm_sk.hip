@@ -2,6 +2,8 @@
 // one translation unit per code width: qgemm_sk_b{2,3,4,5,6,8}.hip).
 #include "qgemm_sk.h"
 
+#include <algorithm>
+
 namespace lxq {
 namespace sk {
 
@@ -22,9 +24,9 @@ extern template LuxStatus launch_bits<8>(const QmmArgs&, int, hipStream_t);
 // against 22.9).  So it runs unsplit from kUnsplitTiles tiles on, and split
 // only where the W-streaming kernel does not apply (K % 1024 != 0).
 constexpr int kUnsplitTiles = 192;
-// at most two blocks per CU; this also bounds the partials: 512 blocks x
-// 32 KiB = 16 MiB
-constexpr int kMaxBlocks = 512;
+// at most one block per CU; this also bounds the partials: 256 blocks x
+// 32 KiB = 8 MiB
+constexpr int kMaxBlocks = 256;
 
 bool applies(int M, int K, int N, int bits, int x_dtype) {
     if (M <= 8 || M > 64 || N <= 0 || (x_dtype != DT_F16 && x_dtype != DT_BF16) || K % kSS != 0) return false;
@@ -37,27 +39,26 @@ bool applies(int M, int K, int N, int bits, int x_dtype) {
     return (N + kCols - 1) / kCols >= kUnsplitTiles || K % 1024 != 0;
 }
 
-// the number of K parts S: 1 from kUnsplitTiles tiles on; else a divisor of
-// K / 128 leaving at least 2 super-steps per part, the smallest that gives
-// kUnsplitTiles blocks without passing kMaxBlocks (else the largest below
-// kMaxBlocks), lowered until the workspace fits `cap`
+// the number of K parts S: 1 from kUnsplitTiles tiles on; else one block per
+// CU, but no more than sqrt(0.9 K / 128) parts (each adds a round trip of its
+// sums) of at least 2 super-steps, lowered until the workspace fits `cap`.
+// Parts need not be equal.  us per launch, against divisors of K / 128 that
+// gave at least kUnsplitTiles blocks: K = 11008 (86 super-steps: 2 parts, 64
+// blocks), N = 4096, 4-bit M = 16 / 32 / 64 31.5 / 32.8 / 44.8 -> 16.1 / 17.4 /
+// 23.7 (8 parts); K = 13440, N = 1000, 8-bit M = 64 39.7 -> 26; K = 3584, N =
+// 4096, 3-bit M = 64 (7 parts) 20.3 -> 18.8 (5); K = 2816, N = 8192, 8-bit M =
+// 20 14.7 -> 12.5 (4).  More blocks than CUs lose: K = 13824, N = 5120, M = 64
+// 29.2 (6 parts, 240 blocks) against 40.6 (7, 280).
 int choose_split(int M, int K, int N, size_t cap) {
     static_assert(kUnsplitTiles <= kMaxSplitTiles, "split tiles have counter slots");
     const int tiles = (N + kCols - 1) / kCols, steps = K / kSS;
     if (tiles >= kUnsplitTiles) return 1;
-    int S = 1;
-    for (int d = 2; d <= steps / 2; d++) {
-        if (steps % d != 0) continue;
-        if (tiles * d > kMaxBlocks) break;
-        S = d;
-        if (tiles * d >= kUnsplitTiles) break;
-    }
-    while (S > 1 && ws_bytes(S, M, N) > cap) {
-        int d = S - 1;
-        while (d > 1 && steps % d != 0) d--;
-        S = d;
-    }
-    return S;
+    int S = std::min(steps / 2, kMaxBlocks / tiles);
+    while (S > 1 && (10 * S * S > 9 * steps || ws_bytes(S, M, N) > cap)) S--;
+    // two short parts save less than their meeting costs: three, or none (K =
+    // 896, N = 300, M = 33: 1 / 2 / 3 parts 9.7 / 10.5 / 9.4)
+    if (S == 2 && steps < 12) S = steps >= 6 && 3 * tiles <= kMaxBlocks && ws_bytes(3, M, N) <= cap ? 3 : 1;
+    return S < 1 ? 1 : S;
 }
 
 }  // namespace sk

@@ -1135,6 +1135,24 @@ def test_lds_gemm_k_parts(ctx, oracle, bits, M, K, N, gs, xd, sbd, od, act):
                  f"K parts b{bits} M{M} K{K} N{N}")
 
 
+@pytest.mark.parametrize("bits", BITS)
+@pytest.mark.parametrize("M,K,N,gs,xd,sbd,od", [(33, 896, 300, 64, F16, F16, F32),   # 7 super-steps in 3 parts
+                                                (64, 11008, 260, 128, BF16, BF16, F32),  # 86 in 8
+                                                (12, 3200, 4097, 32, F16, F32, F16)])   # 25 in 4, one ragged tile
+def test_split_k_gemm_uneven_parts(ctx, oracle, bits, M, K, N, gs, xd, sbd, od):
+    """The split-K small-M GEMM with K parts of different lengths (fewer
+    super-steps than the loads in flight among them), twice."""
+    O = oracle
+    assert ctx.kernel_name(M, K, N, gs, bits, xd, sbd, od, KERNELS["gemm"]) == "qgemm_sk_kernel"
+    x, w_q, s, b, _ = O.make_problem(M, K, N, bits, gs, xd, sbd, seed=8500 + M + bits)
+    print(f"[case] uneven parts M={M} K={K} N={N} b{bits}", flush=True)
+    ys = [run(ctx, x, w_q, s, b, M, K, N, gs, bits, xd, sbd, od, KERNELS["gemm"]) for _ in range(2)]
+    assert np.array_equal(ys[0], ys[1])
+    rows = np.array([0, M - 1])
+    want = O.quantized_matmul(np.ascontiguousarray(x[rows]), w_q, s, b, 2, K, N, gs, bits, xd, sbd, od, w_round=xd)
+    check_output(O, np.ascontiguousarray(ys[0][rows]), want, od, f"uneven parts b{bits} M{M} K{K} N{N}")
+
+
 def test_f32_gemm_special_values(ctx, oracle):
     """An infinity or a NaN in a row of x reaches that row's outputs and no
     other, and x of 2^120, all mantissa bits set, stays finite in its three
