@@ -315,8 +315,10 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
             }
             const int g = ((s & ((1 << gws) - 1)) * BK + 32 * kg) >> gshift;  // group within the window
             const uint8_t* ss = lds + L::kScales + (wi & 1) * L::kWindow + col * L::kScaleRow + g * kSb;
-            sc[t] = sb_f(ss);
-            bi[t] = fmaf(sc[t], C, sb_f(ss + BN * L::kScaleRow));
+            // 32 codes past K (zeros of x): no scale of the next row or the tail
+            const bool in = s * BK + 32 * kg < K;
+            sc[t] = in ? sb_f(ss) : 0.f;
+            bi[t] = in ? fmaf(sc[t], C, sb_f(ss + BN * L::kScaleRow)) : 0.f;
         }
         store_codes(o, stage ^ 1);
         float sum[XL], big = 0.f;

@@ -1172,3 +1172,24 @@ def test_f32_gemm_special_values(ctx, oracle):
     assert np.isfinite(y[11]).all()
     rest = [m for m in range(M) if m not in (2, 7, 9, 11)]
     assert np.array_equal(y[rest], clean[rest])
+
+
+@pytest.mark.parametrize("xd", [F32, F16])
+def test_group_gemm_rows_of_scales_stay_apart(ctx, oracle, xd):
+    """K % 128 == 64: the last step's second half lies past K, where the
+    scale window holds the next row's scales.  A row of NaN scales reaches its
+    own column only."""
+    from mlx_amd import runtime
+    O = oracle
+    M, K, N = 40, 192, 7
+    x, w_q, s, b, _ = O.make_problem(M, K, N, 4, 64, xd, F32, seed=5)
+    clean = runtime.run_quantized_matmul(ctx, x, w_q, s, b, M, K, N, 64, 4, xd, F32, F32)
+    s2, b2 = s.copy(), b.copy()
+    s2[3], b2[3] = np.nan, np.inf
+    assert ctx.kernel_name(M, K, N, 64, 4, xd, F32, F32) == "qgemm_grp_kernel"
+    print(f"[case] group gemm NaN scale row x={xd}", flush=True)
+    y = runtime.run_quantized_matmul(ctx, x, w_q, s2, b2, M, K, N, 64, 4, xd, F32, F32)
+    rest = [n for n in range(N) if n != 3]
+    assert np.isnan(y[:, 3]).all()
+    assert np.array_equal(y[:, rest], clean[:, rest])
+
