@@ -16,14 +16,16 @@ __device__ __forceinline__ uint32_t row_code(const uint32_t* __restrict__ row, i
 }
 
 // Dequantizer.  Rows of codes, scales and outputs are each contiguous over the
-// whole [N, K] matrix (K is a multiple of the group size), so chunk t = the 8
-// codes 8t .. 8t+7 is BITS bytes at byte t * BITS of w_q, 8 outputs at element
-// 8t, and lies in one group.  Lane = chunk: a wave reads 64 * BITS contiguous
-// bytes and writes 1 KB of 16-bit (2 KB of f32) output in 16-byte stores.
+// whole [N, K] matrix (K is a multiple of the group size), so chunk t = the CH
+// codes CH t .. CH t + CH - 1 starts at bit CH t BITS of w_q, fills 16 bytes of
+// the output (CH = 8 of 16-bit, 4 of f32 outputs) and lies in one group.  Lane
+// = chunk: a wave reads contiguous codes and writes 1 KB.
 // Bound by HBM, by the output above all (117 of 150 MB at N = 14336, K = 4096,
 // 4-bit, f16); U chunks per lane, 256 apart, put U code and scale loads in
 // flight before the first store.  One lane per code, a 64-bit division per
-// code and 2-byte stores took 149 us at that size (1.0 TB/s).
+// code and 2-byte stores took 149 us at that size (1.0 TB/s), this 30.4 (5.0);
+// f32 outputs (3-bit, group 32) as two 16-byte halves per lane, 32 bytes
+// apart, 72 us, as one 60.7 (4.4).
 template <int SB>
 __device__ __forceinline__ float sb_at(const void* p, size_t i) {
     if constexpr (SB == DT_F32) return static_cast<const float*>(p)[i];
@@ -46,6 +48,8 @@ template <int BITS, int SB, int OT, int U>
 __global__ __launch_bounds__(256) void dequant_kernel(const uint32_t* __restrict__ wq, const void* __restrict__ sc,
                                                       const void* __restrict__ bi, void* __restrict__ out,
                                                       size_t chunks, int gshift) {
+    constexpr int CH = OT == DT_F32 ? 4 : 8;
+    constexpr int CB = CH * BITS;  // bits of a chunk
     typedef uint32_t o4 __attribute__((ext_vector_type(4)));
     const size_t t0 = (size_t)blockIdx.x * (256 * U) + threadIdx.x;
     uint32_t lo[U], hi[U];
@@ -53,19 +57,21 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint32_t* __restrict
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const size_t t = t0 + 256 * u < chunks ? t0 + 256 * u : chunks - 1;
-        // the chunk's 8 BITS bits in the low end of hi:lo; where they are not
-        // whole words, from the two words they start in (up to 16 + 48 bits:
-        // the second word may lie past w_q, in its readable tail)
-        const size_t byte = t * BITS;
-        if constexpr (BITS == 2) {
+        // the chunk's bits in the low end of hi:lo; where they are not whole
+        // words, from the two words they start in (up to 16 + 48 bits: the
+        // second word may lie past w_q, in its readable tail)
+        if constexpr (CB == 8) {
+            lo[u] = reinterpret_cast<const uint8_t*>(wq)[t];
+        } else if constexpr (CB == 16) {
             lo[u] = reinterpret_cast<const uint16_t*>(wq)[t];
-        } else if constexpr (BITS == 4) {
+        } else if constexpr (CB == 32) {
             lo[u] = wq[t];
         } else {
-            const u32x2 v = *reinterpret_cast<const u32x2*>(wq + (byte >> 2));
-            const uint32_t sh = ((uint32_t)byte & 3u) * 8u;
-            lo[u] = BITS == 8 ? v.x : __builtin_amdgcn_alignbit(v.y, v.x, sh);
-            hi[u] = BITS == 8 ? v.y : v.y >> sh;
+            const size_t bit = t * CB;
+            const u32x2 v = *reinterpret_cast<const u32x2*>(wq + (bit >> 5));
+            const uint32_t sh = (uint32_t)bit & 31u;
+            lo[u] = CB == 64 ? v.x : __builtin_amdgcn_alignbit(v.y, v.x, sh);
+            hi[u] = CB == 64 ? v.y : v.y >> sh;
         }
         const size_t g = t >> gshift;
         s[u] = sb_at<SB>(sc, g);
@@ -75,9 +81,9 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint32_t* __restrict
     for (int u = 0; u < U; u++) {
         const size_t t = t0 + 256 * u;
         if (t >= chunks) return;
-        float v[8];
+        float v[CH];
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
+        for (int i = 0; i < CH; i++) {
             constexpr uint32_t mask = (1u << BITS) - 1u;
             const int bit = i * BITS;
             const uint32_t q = bit + BITS <= 32 ? (lo[u] >> bit) & mask
@@ -85,13 +91,12 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint32_t* __restrict
                                                 : __builtin_amdgcn_alignbit(hi[u], lo[u], bit) & mask;
             v[i] = fmaf(s[u], (float)q, b[u]);
         }
-        o4* o = static_cast<o4*>(out) + t * (OT == DT_F32 ? 2 : 1);
+        o4* o = static_cast<o4*>(out) + t;
         if constexpr (OT == DT_F32) {
             typedef float f4 __attribute__((ext_vector_type(4)));
-            o[0] = __builtin_bit_cast(o4, f4{v[0], v[1], v[2], v[3]});
-            o[1] = __builtin_bit_cast(o4, f4{v[4], v[5], v[6], v[7]});
+            *o = __builtin_bit_cast(o4, f4{v[0], v[1], v[2], v[3]});
         } else {
-            o[0] = o4{cvt_pk<OT>(v[0], v[1]), cvt_pk<OT>(v[2], v[3]), cvt_pk<OT>(v[4], v[5]), cvt_pk<OT>(v[6], v[7])};
+            *o = o4{cvt_pk<OT>(v[0], v[1]), cvt_pk<OT>(v[2], v[3]), cvt_pk<OT>(v[4], v[5]), cvt_pk<OT>(v[6], v[7])};
         }
     }
 }
@@ -262,9 +267,10 @@ LuxStatus launch_dequant_b(const uint32_t* wq, const void* sc, const void* bi, v
 LuxStatus launch_dequantize(const uint32_t* wq, const void* scales, const void* biases, void* out,
                             int N, int K, int group_size, int bits, int sb_dtype, int out_dtype,
                             hipStream_t st) {
-    const size_t chunks = (size_t)N * K / 8;  // group sizes are 32, 64 and 128, so K % 8 == 0
+    const int ch = out_dtype == DT_F32 ? 4 : 8;  // codes per chunk; group sizes are 32, 64 and 128, so K % 8 == 0
+    const size_t chunks = (size_t)N * K / ch;
     if (chunks == 0) return LuxStatus::Ok;
-    const int gshift = group_size == 32 ? 2 : group_size == 64 ? 3 : 4;  // chunks per group, log2
+    const int gshift = (group_size == 32 ? 5 : group_size == 64 ? 6 : 7) - (ch == 4 ? 2 : 3);  // chunks per group, log2
     switch (bits) {
     case 2: return launch_dequant_b<2>(wq, scales, biases, out, chunks, gshift, sb_dtype, out_dtype, st);
     case 3: return launch_dequant_b<3>(wq, scales, biases, out, chunks, gshift, sb_dtype, out_dtype, st);
