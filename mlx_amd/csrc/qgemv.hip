@@ -32,13 +32,17 @@ static LuxStatus launch_mx_bits(const QmmArgs& a, hipStream_t st) {
 // 12.7 / 12.7 / 13.0 / 13.2 / 19.5 against 10.9 / 13.2 / 26.3 / 53.3 / 108; K
 // = 4096, N = 14336, M = 8 / 16 / 128 27.8 / 27.1 / 72.5 against 30.2 / 60.2 /
 // 470; 3-bit K = 14336, N = 4096, M = 16 31 against 145; 5-bit K = 640, N =
-// 1000, M = 16 10.4 against 66.7.  The whole-line kernel keeps its class of up
-// to 16 rows of 3/5/6-bit codes at K <= 4096.
+// 1000, M = 16 10.4 against 66.7.  3/5/6-bit codes at K <= 4096 keep the
+// whole-line kernel's class: up to 16 rows of wide layers (N > 8192) and up to
+// 8 of narrow ones (below 9 tiles of 128 columns).
 static bool grp_f32(const QmmArgs& a) {
     const bool irregular = a.bits == 3 || a.bits == 5 || a.bits == 6;
     const int mx_step = 16 * (a.K > 8192 ? 16 : a.K > 4096 ? 8 : 4);
     const bool rows = irregular || a.K > 16384 || a.K % mx_step != 0;
-    return a.M >= (!rows ? 9 : irregular && a.K <= 4096 ? 17 : 5);
+    if (!rows) return a.M >= 9;
+    if (irregular && a.K <= 4096)
+        return a.M > 16 || (a.N <= 8192 && a.M >= (a.N >= 9 * 128 ? 5 : 9));
+    return a.M >= 5;
 }
 
 // Whether 16-bit x that no M-wide kernel takes runs on the group-wise GEMM
