@@ -24,10 +24,13 @@
 // an odd count: its partner has already counted in -- it is resident and
 // past its K loop -- so it waits for the flag to equal the epoch, adds the
 // stored sums to its own (one fp32 addition per value, the same whichever
-// half is first) and stores y.  Nothing is reset: a flag from an earlier
-// launch holds an older epoch and never satisfies a later wait, and a wait
-// that gives up (a bounded number of polls) leaves the counts consistent for
-// the next launch.
+// half is first) and stores y; having seen the flag, which nobody else waits
+// for, it lowers it.  The counts are never reset.  A launch replayed from a
+// graph carries the same epoch each time: a flag left raised would let the
+// second half of a later replay read the earlier one's sums.  Between launches
+// of different epochs an older flag satisfies no wait.  A wait that gives up
+// (a bounded number of polls) leaves the counts consistent for the next
+// launch.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -80,14 +83,15 @@ __device__ __forceinline__ void publish(void* ws, int st, uint32_t epoch) {
 }
 
 // One thread: wait (s_sleep between polls, at most 2^22 polls, ~0.3 s)
-// for the first half's flag; false if it never came.
+// for the first half's flag, and lower it; false if it never came.
 __device__ __forceinline__ bool wait_partner(void* ws, int st, uint32_t epoch) {
-    const uint32_t* f = static_cast<const uint32_t*>(ws) + kHalfFlagWord + st;
+    uint32_t* f = static_cast<uint32_t*>(ws) + kHalfFlagWord + st;
     uint32_t polls = 0;
     while (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != epoch) {
         if (++polls >= (1u << 22)) return false;
         __builtin_amdgcn_s_sleep(2);
     }
+    __hip_atomic_store(f, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return true;
 }
 

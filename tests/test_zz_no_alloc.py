@@ -176,6 +176,56 @@ def test_noalloc_graph_capture(ctx, oracle):
         hip.ck(hip.L.hipStreamDestroy(stream), "hipStreamDestroy")
 
 
+@pytest.mark.parametrize("call", [
+    (2000, 1024, 4360, 4, 64, BF16, BF16, BF16, 2),  # 32 tiles in K halves
+    (100, 1536, 300, 3, 64, F16, F16, F16, 0),       # K parts, summed by a second launch
+    (40, 4160, 300, 4, 64, BF16, BF16, F32, 0),      # group-wise GEMM, K parts
+], ids=["halves", "parts", "group"])
+def test_noalloc_graph_new_inputs(ctx, oracle, call):
+    """A captured call whose parts meet in the scratch, replayed with another
+    x each time (copied over the captured one between replays): every replay
+    equals the context op on that x bit for bit."""
+    from mlx_amd import runtime
+    O = oracle
+    f = _entry()
+    hip = _Hip()
+    M, K, N, bits, gs, xd, sbd, od, kern = call
+    _, w_q, s, b, _ = O.make_problem(M, K, N, bits, gs, xd, sbd, seed=770)
+    xs = [O.make_problem(M, K, 32, bits, gs, xd, sbd, seed=771 + i)[0] for i in range(3)]
+    stream = ctypes.c_void_p()
+    hip.ck(hip.L.hipStreamCreate(ctypes.byref(stream)), "hipStreamCreate")
+    ptrs = [hip.upload(np.ascontiguousarray(a)) for a in (xs[0], w_q, s, b)]
+    more = [hip.upload(np.ascontiguousarray(a)) for a in xs]
+    out = hip.alloc(M * N * runtime.esize(od))
+    graph, exe = ctypes.c_void_p(), ctypes.c_void_p()
+    try:
+        assert f(*ptrs, out, M, K, N, gs, bits, xd, sbd, od, kern, stream) == 0
+        hip.ck(hip.L.hipStreamSynchronize(stream), "hipStreamSynchronize")
+        hip.ck(hip.L.hipStreamBeginCapture(stream, 0), "hipStreamBeginCapture")
+        rc = f(*ptrs, out, M, K, N, gs, bits, xd, sbd, od, kern, stream)
+        hip.ck(hip.L.hipStreamEndCapture(stream, ctypes.byref(graph)), "hipStreamEndCapture")
+        assert rc == 0, f"captured noalloc call returned {rc}"
+        hip.ck(hip.L.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, 0), "hipGraphInstantiate")
+        for rep in range(3):
+            print(f"[case] noalloc graph replay {rep} on another x: M={M} K={K} N={N}", flush=True)
+            # device to device (kind 3), waited for before the replay
+            hip.ck(hip.L.hipMemcpy(ptrs[0], more[rep], ctypes.c_size_t(xs[rep].nbytes), 3), "hipMemcpy")
+            hip.ck(hip.L.hipDeviceSynchronize(), "hipDeviceSynchronize")
+            hip.ck(hip.L.hipGraphLaunch(exe, stream), "hipGraphLaunch")
+            hip.ck(hip.L.hipStreamSynchronize(stream), "hipStreamSynchronize")
+            got = hip.download(out, runtime.np_dtype(od), (M, N))
+            want = runtime.run_quantized_matmul(ctx, xs[rep], w_q, s, b, M, K, N, gs, bits, xd, sbd, od, kern)
+            assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), f"replay {rep} differs"
+    finally:
+        if exe.value:
+            hip.L.hipGraphExecDestroy(exe)
+        if graph.value:
+            hip.L.hipGraphDestroy(graph)
+        for p in ptrs + more + [out]:
+            hip.free(p)
+        hip.ck(hip.L.hipStreamDestroy(stream), "hipStreamDestroy")
+
+
 def test_noalloc_errors():
     """Errors come back before any device work: null pointers, a bad shape.
     The pointers are real (small) device allocations, so a check that ran
