@@ -107,9 +107,13 @@ void launch_parts(const QmmArgs& a, int mtiles, int nsplit, hipStream_t st) {
 
 // K parts for a shape with few tiles (1: none, whole tiles or halves of a
 // split round) of KT steps, at most `most`, the cheapest in twentieths of a
-// us: a step costs `step` (LDS-dequant GEMM: 20), a part's 128 KiB 1 (stored
-// and loaded by all CUs together), the second launch 60, the meeting of two
-// halves 100.  Same box, us per launch, halves or whole tiles / K parts
+// us: a step of the longest part costs `step` (LDS-dequant GEMM: 20), a part's
+// 128 KiB 1 (stored and loaded by all CUs together), the second launch 60, the
+// meeting of two halves 100.  Parts are whole units of KT / most steps, so
+// counts that do not divide them leave one part longer than KT / S: priced at
+// KT / S they took M = 330, K = 1024, N = 1778, 6-bit as 3 parts of 1, 1 and 2
+// units, 19.6 us, against 18.2 as 4; M = 370, K = 2048, N = 675, 6-bit 7 parts
+// 20.1, 8 17.4; M = 75, K = 6144, N = 393, 3-bit 20 parts 17.6, 24 15.0.  Same box, us per launch, halves or whole tiles / K parts
 // (tiles, parts): LDS-dequant GEMM M = 509, K = 11008, N = 4096, 6-bit, GELU
 // (64, 4) 173 / 69; M = 512, K = N = 4096, 6-bit (64, 4) 41.4 / 35.6; M = 128,
 // K = N = 4096, 3-bit (32, 8) 38.7 / 24.8, N = 10000 (79, 3) 40.6 / 34.6; M =
@@ -125,7 +129,7 @@ inline int k_parts(int tiles, int KT, int most, bool halves, int step, const Qmm
                              (int)((a.ws_bytes - split::kPartOffset) / ((size_t)tiles * kTileBytes)));
     int best = 1, least = halves && a.epoch != 0u ? step * KT / 2 + 100 : step * KT;
     for (int S = 2; S <= cap; S++) {
-        const int cost = (step * KT + S - 1) / S + 60 + tiles * S;
+        const int cost = step * (KT / most) * ((most + S - 1) / S) + 60 + tiles * S;
         if (cost < least) { least = cost; best = S; }
     }
     return best;
