@@ -74,14 +74,14 @@ def code_objects(tmp_path_factory):
     return cos
 
 
-@pytest.fixture(scope="module")
-def disassembly(code_objects):
+def _disassemble(code_objects, kernels):
+    """{kernel symbol: its instructions} of the kernels whose names hold one of `kernels`."""
     objdump = _tool("llvm-objdump")
     out = {}
     for co in code_objects:
         syms = subprocess.run([objdump, "-t", str(co)], check=True, capture_output=True, text=True).stdout
         names = [ln.split()[-1] for ln in syms.splitlines()
-                 if " .text" in ln and any(k in ln for k in KERNELS + (LINE, MX, Q4, SK)) and not ln.endswith(".kd")]
+                 if " .text" in ln and any(k in ln for k in kernels) and not ln.endswith(".kd")]
         if not names:
             continue
         dis = subprocess.run([objdump, "-d", "--mcpu=gfx950", "--disassemble-symbols=" + ",".join(names), str(co)],
@@ -95,6 +95,11 @@ def disassembly(code_objects):
             elif cur and ln.strip():
                 out[cur].append(ln.strip())
     return out
+
+
+@pytest.fixture(scope="module")
+def disassembly(code_objects):
+    return _disassemble(code_objects, KERNELS + (LINE, MX, Q4, SK))
 
 
 def test_weight_loads_precede_their_wait(disassembly):
@@ -222,3 +227,18 @@ def test_no_kernel_spills_to_scratch(code_objects):
                 bad.append(f"{name.group(1)}: {priv.group(1)} bytes of scratch per lane")
     assert seen > 100, f"only {seen} kernels found in the code objects' metadata"
     assert not bad, f"{len(bad)} kernels spill:\n" + "\n".join(bad[:10])
+
+
+def test_matmul_stores_whole_rows(code_objects):
+    """The dense matmul's micro-tiles of 2 or 4 columns leave a row per store
+    (value by value, lanes RN columns apart, they cost up to half as much again
+    as the launch where K is short)."""
+    seen = 0
+    for name, lines in _disassemble(code_objects, ["matmul_kernelI"]).items():
+        m = re.search(r"MmTileILi\d+ELi\d+ELi\d+ELi(\d+)E", name)
+        if not m or int(m.group(1)) == 1:
+            continue
+        seen += 1
+        want = {2: "global_store_dwordx2", 4: "global_store_dwordx4"}[int(m.group(1))]
+        assert any(t.startswith(want) for t in lines), f"{name}: no {want}"
+    assert seen == 4
