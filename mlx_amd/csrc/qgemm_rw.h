@@ -137,6 +137,13 @@ __device__ __forceinline__ void barrier() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// the barrier behind which other waves read what this wave wrote to LDS, or
+// overwrite what it reads: the builtin waits for neither
+__device__ __forceinline__ void barrier_lds() {
+    wait_lgkm0();
+    barrier();
+}
+
 // global -> LDS: lane l copies 16 bytes from sbase + voff to LDS m0 + 16 l
 __device__ __forceinline__ void dma16(uint32_t m0v, const void* sbase, uint32_t voff) {
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(m0v), "v"(voff), "s"(sbase) : "memory", "m0");
@@ -584,7 +591,7 @@ __device__ __forceinline__ void hand_half(uint8_t* hs, int rs, const f32x16 (&ac
     constexpr int I0 = P * C::MT / 2, I1 = I0 + C::MT / 2, kHalf = kHand<C> / 2;
     if (ep.out_dt == DT_BF16) stage16<C, EPI, DT_BF16, I0, I1>(hs, rs, acc, ep, n0, N, wave, c, h);
     else stage16<C, EPI, DT_F16, I0, I1>(hs, rs, acc, ep, n0, N, wave, c, h);
-    barrier();
+    barrier_lds();
 #pragma unroll
     for (int i = 0; i < kHalf; i++) {
         const int q = tid + i * C::kThreads;
@@ -681,19 +688,19 @@ __global__ __launch_bounds__(C::kThreads, 1) void qgemm_rw_kernel(
             next_unit(un);
             uint8_t* hs = lds + C::kLds;
             hand_half<C, EPI, 0>(hs, rs, acc, ep, no, N, wave, c, h, tid, val);
-            barrier();
+            barrier_lds();  // half 0 is read before half 1 overwrites it
             hand_half<C, EPI, 1>(hs, rs, acc, ep, no, N, wave, c, h, tid, val);
         } else {
             // the tile in the rings in one pass, then the next unit's transfers
             if (ep.out_dt == DT_BF16) stage16<C, EPI, DT_BF16>(lds, rs, acc, ep, no, N, wave, c, h);
             else stage16<C, EPI, DT_F16>(lds, rs, acc, ep, no, N, wave, c, h);
-            barrier();
+            barrier_lds();
 #pragma unroll
             for (int i = 0; i < kHand<C>; i++) {
                 const int q = tid + i * C::kThreads;
                 val[i] = *reinterpret_cast<const u4*>(lds + (q >> 5) * rs + (q & 31) * 16);
             }
-            barrier();
+            barrier_lds();
             next_unit(un);
         }
         // the stores: chunks past M or N (whole chunks, N % 8 == 0) get an
@@ -725,7 +732,7 @@ __global__ __launch_bounds__(C::kThreads, 1) void qgemm_rw_kernel(
             static_cast<uint8_t*>(ws) + split::kPartOffset, 0, (int)(nslots * kSlot), 0x00020000);
         barrier();
         if (tid == 0) *word = split::arrive_first(ws, st) ? 1u : 0u;
-        barrier();
+        barrier_lds();
         const uint32_t slot = (uint32_t)st * kSlot;
         if (*word == 1u) {
 #pragma unroll
@@ -743,7 +750,7 @@ __global__ __launch_bounds__(C::kThreads, 1) void qgemm_rw_kernel(
             return;
         }
         if (tid == 0) *word = split::wait_partner(ws, st, epoch) ? 2u : 3u;
-        barrier();
+        barrier_lds();
         const float fail = *word == 2u ? 0.f : __builtin_nanf("");
 #pragma unroll
         for (int q = 0; q < kVec; q++) {
@@ -773,7 +780,7 @@ __global__ __launch_bounds__(C::kThreads, 1) void qgemm_rw_kernel(
         barrier();
         if (ep.out_dt == DT_BF16) stage16<C, EPI, DT_BF16>(lds, rs, acc, ep, n0, N, wave, c, h);
         else stage16<C, EPI, DT_F16>(lds, rs, acc, ep, n0, N, wave, c, h);
-        barrier();
+        barrier_lds();
         // row r: BN * 2 bytes = 32 16-byte chunks
         for (int q = tid; q < BM * 32; q += C::kThreads) {
             const int rl = q / 32, ch = q % 32;
@@ -812,7 +819,7 @@ __global__ __launch_bounds__(C::kThreads, 1) void qgemm_rw_kernel(
                     *reinterpret_cast<float*>(lds + ml * rs + (wave * C::WN + 32 * tt + c) * 4) = acc[i][tt][v];
                 }
         }
-        barrier();
+        barrier_lds();
 #pragma unroll 1
         for (int rl = tid / 32; rl < prow; rl += C::kThreads / 32) {
             const int r = ps * prow + rl, m = m0 + r;

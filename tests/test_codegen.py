@@ -242,3 +242,27 @@ def test_matmul_stores_whole_rows(code_objects):
         want = {2: "global_store_dwordx2", 4: "global_store_dwordx4"}[int(m.group(1))]
         assert any(t.startswith(want) for t in lines), f"{name}: no {want}"
     assert seen == 4
+
+
+def test_lds_writes_are_waited_for_before_a_barrier(code_objects, disassembly):
+    """The kernels that issue s_barrier themselves never reach one with LDS
+    writes in flight, in program order: the instruction waits for nothing, and
+    what other waves read behind it must have been written."""
+    seen, bad = 0, []
+    rw = _disassemble(code_objects, ["qgemm_rw_kernel"])
+    assert rw, "qgemm_rw_kernel not found in the plugin"
+    for name, lines in {**disassembly, **rw}.items():
+        pending = barriers = 0
+        for t in lines:
+            if t.startswith("ds_write"):
+                pending = 1
+            elif re.search(r"s_waitcnt\b.*\blgkmcnt\(0\)", t):
+                pending = 0
+            elif t.startswith("s_barrier"):
+                barriers += 1
+                if pending:
+                    bad.append(name)
+                    break
+        seen += barriers > 0
+    assert seen > 100, f"only {seen} kernels with a barrier found in the plugin"
+    assert not bad, f"{len(bad)} kernels:\n" + "\n".join(bad[:10])
