@@ -626,7 +626,8 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_kernel(
         // never published (bounded wait)
         if (tid == 0) *word = split::wait_partner(ws, st, epoch) ? 2u : 3u;
         __syncthreads();
-        const float fail = *word == 2u ? 0.f : __builtin_nanf("");
+        const bool seen = *word == 2u;
+        const float fail = seen ? 0.f : __builtin_nanf("");
         v4 o[16];
 #pragma unroll
         for (int q = 0; q < 16; q++)
@@ -641,6 +642,7 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_kernel(
             a[v + 2] += __uint_as_float(o[q].z) + fail;
             a[v + 3] += __uint_as_float(o[q].w) + fail;
         }
+        if (tid == 0 && seen) split::lower(ws, st);
     }
 
     // ---- output: the fp32 tile through LDS (free once every wave is past its

@@ -751,7 +751,8 @@ __global__ __launch_bounds__(C::kThreads, 1) void qgemm_rw_kernel(
         }
         if (tid == 0) *word = split::wait_partner(ws, st, epoch) ? 2u : 3u;
         barrier_lds();
-        const float fail = *word == 2u ? 0.f : __builtin_nanf("");
+        const bool seen = *word == 2u;
+        const float fail = seen ? 0.f : __builtin_nanf("");
 #pragma unroll
         for (int q = 0; q < kVec; q++) {
             const u4 o = __builtin_amdgcn_raw_buffer_load_b128(pr, voff, slot + (uint32_t)q * (C::kThreads * 16u),
@@ -763,6 +764,7 @@ __global__ __launch_bounds__(C::kThreads, 1) void qgemm_rw_kernel(
             a[v + 2] += __uint_as_float(o.z) + fail;
             a[v + 3] += __uint_as_float(o.w) + fail;
         }
+        if (tid == 0 && seen) split::lower(ws, st);
     }
 
     // ---- output: lane holds column c of each 32 x 32 tile, VGPR v row
