@@ -645,12 +645,39 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_kernel(
         if (tid == 0 && seen) split::lower(ws, st);
     }
 
-    // ---- output: the fp32 tile through LDS (free once every wave is past its
-    // K loop; 32x32 accumulator layout: lane holds column (lane % 32), VGPR v
-    // row 8 (v / 4) + 4 (lane / 32) + v % 4), then whole 16-byte chunks of
-    // rows.  The loop stays rolled: unrolled, the activations' code (64 copies
-    // of erf or exp per thread) ran from cold instruction cache misses and
-    // took 20 us at M = 509, N = 4096 with GELU ----
+    // ---- output (32x32 accumulator layout: lane holds column (lane % 32),
+    // VGPR v row 8 (v / 4) + 4 (lane / 32) + v % 4).  Plain values leave the
+    // registers one by one, 32 columns of a row side by side: 64 stores per
+    // thread for any N, where the LDS tile below took longer (M = 895, K =
+    // 256, 4-bit, f32 y, us per launch: N = 2048 9.6 against 11.0, N = 2045
+    // 9.8 against 12.9; M = 511, K = 1024, 2-bit, bf16 y: N = 4183 21.5
+    // against 26.4) ----
+    if constexpr (!EPI) {
+        if (nsplit == 1) {
+            const int ncol = t.n0 + wn * 64 + (lane & 31), mrow = m0 + wm * 64 + 4 * (lane >> 5);
+            auto store = [&](auto* yo, auto value) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++) {
+                        const int n = ncol + j * 32;
+#pragma unroll
+                        for (int v = 0; v < 16; v++) {
+                            const int m = mrow + i * 32 + 8 * (v >> 2) + (v & 3);
+                            if (m < M && n < N) yo[(size_t)m * N + n] = value(acc[i][j][v]);
+                        }
+                    }
+            };
+            const bool bf = ep.out_dt == DT_BF16;
+            if (ep.out_dt == DT_F32) store(static_cast<float*>(y), [](float o) { return o; });
+            else store(static_cast<uint16_t*>(y), [&](float o) { return bf ? f32_to_bf16(o) : f32_to_f16(o); });
+            return;
+        }
+    }
+    // The others go through LDS (free once every wave is past its K loop),
+    // then in whole chunks of 8 columns.  The loop stays rolled: unrolled, the
+    // activations' code (64 copies of erf or exp per thread) ran from cold
+    // instruction cache misses and took 20 us at M = 509, N = 4096 with GELU
     __syncthreads();
     float* tile_out = reinterpret_cast<float*>(lds);
     {
@@ -663,10 +690,10 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_kernel(
                 for (int v = 0; v < 16; v++) d[(i * 32 + 8 * (v >> 2) + (v & 3)) * kOutRow + j * 32] = acc[i][j][v];
     }
     __syncthreads();
-    // thread: columns 8 (tid % 16) ..+8 of rows tid / 16, + 32, ...
-    const int nl = tid % (BN / 8) * 8, n = t.n0 + nl;
     if (nsplit > 1) {
-        // a K part: its tile of sums, row by row, for parts_kernel
+        // a K part: its tile of sums, row by row, for parts_kernel; thread:
+        // columns 8 (tid % 16) ..+8 of rows tid / 16, + 32, ...
+        const int nl = tid % (BN / 8) * 8;
         float* d = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + split::kPartOffset) +
                    (size_t)(tile * nsplit + part) * (BM * BN);
 #pragma unroll 4
@@ -679,14 +706,19 @@ __global__ __launch_bounds__(kThreads, 2) void qgemm_kernel(
         }
         return;
     }
-    if (n >= N) return;
-    const RowOut out(y, N, n, ep);
+    if constexpr (EPI) {
+        // thread: a chunk of 8 columns of rows tid / w, + kThreads / w, ...
+        const int w = row_chunks<BN>(N - t.n0);
+        const int nl = tid % w * 8, n = t.n0 + nl;
+        if (n >= N) return;
+        const RowOut out(y, N, n, ep);
 #pragma unroll 1
-    for (int r = tid / (BN / 8); r < BM && m0 + r < M; r += kThreads / (BN / 8)) {
-        float o[8];
+        for (int r = tid / w; r < BM && m0 + r < M; r += kThreads / w) {
+            float o[8];
 #pragma unroll
-        for (int e = 0; e < 8; e++) o[e] = tile_out[r * kOutRow + nl + e];
-        out.store<EPI>(m0 + r, o, ep);
+            for (int e = 0; e < 8; e++) o[e] = tile_out[r * kOutRow + nl + e];
+            out.store<true>(m0 + r, o, ep);
+        }
     }
 }
 

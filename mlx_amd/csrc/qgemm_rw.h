@@ -802,11 +802,8 @@ __global__ __launch_bounds__(C::kThreads, 1) void qgemm_rw_kernel(
     }
     constexpr int rs = BN * 4 + 16;
     constexpr int passes = BM * rs > C::kLds ? 2 : 1, prow = BM / passes;
-    // thread: columns 8 (tid % 32) ..+8 of rows tid / 32, + kThreads / 32, ...
-    const int nl = tid % 32 * 8, n = n0 + nl;
-    const tileout::RowOut out(y, N, n < N ? n : N - 1, ep);
     float* part = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + split::kPartOffset) +
-                  (size_t)(w.tile * nsplit + (nsplit > 1 ? w.part : 0)) * (BM * BN) + nl;
+                  (size_t)(w.tile * nsplit + (nsplit > 1 ? w.part : 0)) * (BM * BN);
 #pragma unroll
     for (int ps = 0; ps < passes; ps++) {
         barrier();
@@ -822,24 +819,37 @@ __global__ __launch_bounds__(C::kThreads, 1) void qgemm_rw_kernel(
                 }
         }
         barrier_lds();
+        if (!EPI || nsplit > 1) {
+            // row r: 64 16-byte chunks (dword-aligned: rows of any N)
+            typedef uint32_t u4d __attribute__((ext_vector_type(4), aligned(4)));
+            for (int q = tid; q < prow * 64; q += C::kThreads) {
+                const int r = ps * prow + q / 64, nl = q % 64 * 4, m = m0 + r, n = n0 + nl;
+                if (m >= M || n >= N) continue;
+                const u4 val = *reinterpret_cast<const u4*>(lds + (q / 64) * rs + nl * 4);
+                float* dst = nsplit > 1 ? part + r * BN + nl : static_cast<float*>(y) + (size_t)m * N + n;
+                if (nsplit > 1 || n + 4 <= N) {
+                    *reinterpret_cast<u4d*>(dst) = val;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 3; e++)
+                        if (n + e < N) reinterpret_cast<uint32_t*>(dst)[e] = val[e];
+                }
+            }
+        } else {
+            // thread: a chunk of 8 columns of rows tid / cw, + kThreads / cw, ...
+            const int cw = tileout::row_chunks<BN>(N - n0);
+            const int nl = tid % cw * 8, n = n0 + nl;
+            if (n >= N) continue;
+            const tileout::RowOut out(y, N, n, ep);
 #pragma unroll 1
-        for (int rl = tid / 32; rl < prow; rl += C::kThreads / 32) {
-            const int r = ps * prow + rl, m = m0 + r;
-            if (m >= M || n >= N) break;
-            const u4* src = reinterpret_cast<const u4*>(lds + rl * rs + nl * 4);
-            const u4 a = src[0], b = src[1];
-            if (nsplit > 1) {
-                u4* d = reinterpret_cast<u4*>(part + (size_t)r * BN);
-                d[0] = a;
-                d[1] = b;
-            } else {
+            for (int rl = tid / cw; rl < prow; rl += C::kThreads / cw) {
+                const int m = m0 + ps * prow + rl;
+                if (m >= M) break;
+                const float* src = reinterpret_cast<const float*>(lds + rl * rs) + nl;
                 float o[8];
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    o[e] = __uint_as_float(a[e]);
-                    o[4 + e] = __uint_as_float(b[e]);
-                }
-                out.store<EPI>(m, o, ep);
+                for (int e = 0; e < 8; e++) o[e] = src[e];
+                out.store<true>(m, o, ep);
             }
         }
     }

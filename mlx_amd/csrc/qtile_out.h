@@ -26,14 +26,19 @@ __device__ __forceinline__ uint32_t pair(float a, float b) {
 }
 
 // 8 columns n .. n + 7 of rows of y, through the output stage: their biases,
-// loaded once, and vector stores where rows keep 16-byte alignment
+// loaded once, and one (16-bit y) or two (f32) 16-byte stores per row.  Rows
+// of any N and y of any alignment its type allows: the stores need no more
+// than that.  Only the chunk that N ends in stores value by value.  (As whole
+// 16-byte chunks where N allowed them, else value by value, every lane 8
+// columns from the next: LDS-dequant GEMM M = 1414, K = 256, N = 4913, 3-bit,
+// GELU 34.6 us, so 24.2; M = 215, K = 256, N = 8377, 4-bit, RELU 22.8 and 13.7.)
 struct RowOut {
+    typedef uint32_t f32x4 __attribute__((ext_vector_type(4), aligned(4)));
+    typedef uint32_t u16x8 __attribute__((ext_vector_type(4), aligned(2)));
     void* y;
     int N, n;
-    bool vec;
     float bias[8];
     __device__ __forceinline__ RowOut(void* y_, int N_, int n_, const Epilogue& ep) : y(y_), N(N_), n(n_) {
-        vec = (((uintptr_t)y) & 15) == 0 && N % (ep.out_dt == DT_F32 ? 4 : 8) == 0 && n + 8 <= N;
 #pragma unroll
         for (int e = 0; e < 8; e++) bias[e] = ep.bias ? load_f(ep.bias, (size_t)min(n + e, N - 1), ep.bias_dt) : 0.f;
     }
@@ -47,25 +52,49 @@ struct RowOut {
             }
         }
         const size_t at = (size_t)m * N + n;
-        if (!vec) {
+        if (ep.out_dt == DT_F32) {
+            float* d = static_cast<float*>(y) + at;
+            if (n + 8 <= N) {
 #pragma unroll
-            for (int e = 0; e < 8; e++)
-                if (n + e < N) store_f(y, at + e, ep.out_dt, o[e]);
-        } else if (ep.out_dt == DT_F32) {
-            t4* d = reinterpret_cast<t4*>(static_cast<float*>(y) + at);
+                for (int e = 0; e < 8; e += 4)
+                    *reinterpret_cast<f32x4*>(d + e) = f32x4{__float_as_uint(o[e]), __float_as_uint(o[e + 1]),
+                                                             __float_as_uint(o[e + 2]), __float_as_uint(o[e + 3])};
+            } else {
 #pragma unroll
-            for (int e = 0; e < 8; e += 4)
-                d[e / 4] = t4{__float_as_uint(o[e]), __float_as_uint(o[e + 1]), __float_as_uint(o[e + 2]),
-                              __float_as_uint(o[e + 3])};
+                for (int e = 0; e < 7; e++)
+                    if (n + e < N) d[e] = o[e];
+            }
+            return;
+        }
+        u16x8 p;
+        if (ep.out_dt == DT_BF16) {
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) p[e / 2] = pair<DT_BF16>(o[e], o[e + 1]);
         } else {
-            t4 p;
 #pragma unroll
-            for (int e = 0; e < 8; e += 2)
-                p[e / 2] = ep.out_dt == DT_BF16 ? pair<DT_BF16>(o[e], o[e + 1]) : pair<DT_F16>(o[e], o[e + 1]);
-            *reinterpret_cast<t4*>(static_cast<uint16_t*>(y) + at) = p;
+            for (int e = 0; e < 8; e += 2) p[e / 2] = pair<DT_F16>(o[e], o[e + 1]);
+        }
+        uint16_t* d = static_cast<uint16_t*>(y) + at;
+        if (n + 8 <= N) {
+            *reinterpret_cast<u16x8*>(d) = p;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 7; e++)
+                if (n + e < N) d[e] = (uint16_t)(p[e / 2] >> (16 * (e & 1)));
         }
     }
 };
+
+// chunks of 8 columns per row of a tile BN wide that has `cols` of them left,
+// to the next power of two (a thread keeps its columns from row to row): a
+// narrow tile's rows go to all the threads (M = 1182, K = 256, N = 15, 4-bit,
+// RELU: as 16 chunks per row, 14 of them idle, 19.6 us, so 9.2)
+template <int BN>
+__device__ __forceinline__ int row_chunks(int cols) {
+    int w = BN / 8;
+    while (w > 1 && w * 4 >= cols) w >>= 1;
+    return w;
+}
 
 // Sum of the K parts: 8 columns of a row per thread, the parts' tiles in part
 // order, then the output stage.  (As the last part's own work at M = 509, K =

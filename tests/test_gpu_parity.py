@@ -1193,3 +1193,42 @@ def test_group_gemm_rows_of_scales_stay_apart(ctx, oracle, xd):
     assert np.isnan(y[:, 3]).all()
     assert np.array_equal(y[:, rest], clean[:, rest])
 
+
+
+@pytest.mark.parametrize("od,act", [(F32, 0), (F16, 0), (F32, 1), (F16, 3)])
+@pytest.mark.parametrize("M,K,N,bits,kernel", [
+    (300, 256, 4, 3, "qgemm_kernel"),        # a tile of less than one chunk of 8 columns
+    (300, 256, 15, 3, "qgemm_kernel"),       # one chunk and 7 columns
+    (300, 256, 261, 3, "qgemm_kernel"),      # a last tile of 5 columns
+    (290, 768, 190, 5, "qgemm_kernel"),      # a last tile of 8 chunks less 2 columns
+    (1300, 1024, 3333, 4, "qgemm_rw_kernel"),  # 154 whole tiles, the last ones 5 columns wide
+    (1300, 1024, 3391, 8, "qgemm_rw_kernel")])  # the last ones 8 chunks less a column
+def test_gemm_rows_of_odd_length(ctx, oracle, M, K, N, bits, kernel, od, act):
+    """Rows of y that keep no alignment, and tiles narrower than their kernel's:
+    the direct stores, the rows through LDS and the fused output stage store
+    every column and nothing past a row."""
+    from mlx_amd import runtime
+    O = oracle
+    assert ctx.kernel_name(M, K, N, 64, bits, F16, F16, od) == kernel
+    x, w_q, s, b, _ = O.make_problem(M, K, N, bits, 64, F16, F16, seed=8600 + N + bits)
+    bias = O.rng_normal(N, seed=8700 + N).astype(np.float32)
+    bufs = [ctx.upload(a) for a in (x, w_q, s, b)]
+    bb = ctx.upload(bias)
+    out = ctx.upload(np.full(M * N + 64, 0x7f, np.uint8).repeat(runtime.esize(od)))
+    print(f"[case] odd rows M={M} K={K} N={N} b{bits} out={od} act={act}", flush=True)
+    try:
+        if act:
+            ctx.quantized_matmul_fused(*bufs, bb, out, M, K, N, 64, bits, F16, F16, F32, od, act)
+        else:
+            ctx.quantized_matmul(*bufs, out, M, K, N, 64, bits, F16, F16, od)
+        raw = out.download(np.uint8, ((M * N + 64) * runtime.esize(od),))
+    finally:
+        for t in bufs + [bb, out]:
+            t.free()
+    assert np.all(raw[M * N * runtime.esize(od):] == 0x7f)
+    y = raw[:M * N * runtime.esize(od)].view(runtime.np_dtype(od)).reshape(M, N)
+    rows = np.unique(np.r_[0, 1, M // 2, M - 1])
+    acc = O.quantized_matmul(np.ascontiguousarray(x[rows]), w_q, s, b, len(rows), K, N, 64, bits, F16, F16, F32,
+                             variant="omp", w_round=F16)
+    want = O.fused_epilogue(acc, bias, F32, act, od) if act else acc if od == F32 else O.from_f32(acc, od)
+    check_output(O, np.ascontiguousarray(y[rows]), want, od, f"odd rows M{M} N{N} b{bits}")
