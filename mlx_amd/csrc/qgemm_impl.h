@@ -737,7 +737,7 @@ LuxStatus launch4_e(const QmmArgs& a, hipStream_t st) {
         const int tiles = mtiles * ntiles;
         // (scale windows of 4 steps; halves of whole windows)
         const int KT = a.K / BK;
-        const int nsplit = k_parts(tiles, KT, KT / 4, KT % 8 == 0, 20, a);
+        const int nsplit = k_parts(tiles, KT, KT / 4, KT % 8 == 0, kLdsPrice, a);
         // the last round's tiles in two K halves where that round is at most
         // half full (each half a whole number of 4-step scale windows)
         const int r = tiles % kCUs;

@@ -873,8 +873,8 @@ LuxStatus launch_e(const QmmArgs& a, hipStream_t st) {
     if (attr != hipSuccess) return LuxStatus::Internal;
     const int mtiles = (a.M + C::BM - 1) / C::BM, ntiles = (a.N + BN - 1) / BN;
     const int tiles = mtiles * ntiles, KT = a.K / BK;
-    // K parts of whole unrolled loops each; a step of the tile costs 0.9 us
-    const int nsplit = tileout::k_parts(tiles, KT, KT / C::kUnroll, (KT / 2) % C::kUnroll == 0, 18, a);
+    // K parts of whole unrolled loops each
+    const int nsplit = tileout::k_parts(tiles, KT, KT / C::kUnroll, (KT / 2) % C::kUnroll == 0, tileout::kRwPrice, a);
     // with whole tiles: the last round's tiles in two K halves where that
     // round is at most half full (each half a whole number of unrolled loops)
     const int r = tiles % kCUs;

@@ -134,31 +134,43 @@ void launch_parts(const QmmArgs& a, int mtiles, int nsplit, hipStream_t st) {
                        a.y, a.M, a.N, a.epi(), mtiles, nsplit);
 }
 
-// K parts for a shape with few tiles (1: none, whole tiles or halves of a
-// split round) of KT steps, at most `most`, the cheapest in twentieths of a
-// us: a step of the longest part costs `step` (LDS-dequant GEMM: 20), a part's
-// 128 KiB 1 (stored and loaded by all CUs together), the second launch 60, the
-// meeting of two halves 100.  Parts are whole units of KT / most steps, so
-// counts that do not divide them leave one part longer than KT / S: priced at
-// KT / S they took M = 330, K = 1024, N = 1778, 6-bit as 3 parts of 1, 1 and 2
-// units, 19.6 us, against 18.2 as 4; M = 370, K = 2048, N = 675, 6-bit 7 parts
-// 20.1, 8 17.4; M = 75, K = 6144, N = 393, 3-bit 20 parts 17.6, 24 15.0.  Same box, us per launch, halves or whole tiles / K parts
-// (tiles, parts): LDS-dequant GEMM M = 509, K = 11008, N = 4096, 6-bit, GELU
-// (64, 4) 173 / 69; M = 512, K = N = 4096, 6-bit (64, 4) 41.4 / 35.6; M = 128,
-// K = N = 4096, 3-bit (32, 8) 38.7 / 24.8, N = 10000 (79, 3) 40.6 / 34.6; M =
-// 100, K = 14336, N = 1000, 3-bit (8, 32) 107 / 22; M = 70, K = 1024, N = 128,
-// 3-bit (1, 4) 15.4 / 10.6; not taken: M = 1024, K = N = 4096, 3-bit (128, 2)
-// 48.9 / 53.7; M = 250, K = 1024, N = 9000, 5-bit (71, 3) 21.8 / 26.2.
-// Register-W GEMM, its parts summed by the last to arrive / by the launch:
+// What a shape's split costs, in eightieths of a us: a K step; the meeting of
+// two halves, and more per tile; the parts' launch, and each part's 128 KiB
+// (stored and loaded by all CUs together), up to 128 parts and past them; the
+// output stage fused into whole tiles or halves instead of that launch.
+struct PartPrice {
+    int step, halves, halves_tile, launch, part, part_past, fused;
+};
+// LDS-dequant GEMM: fitted to 492 launches of 1 to 100 tiles, K = 512 .. 8192,
+// 3-bit (0.3 % above the best split of each in the mean), against which a
+// price of 20 twentieths a step, 100 for halves, 60 for the launch and 1 per
+// part was up to 34 % off.  us, halves or whole tiles / K parts (parts): M =
+// 2045, N = 507, K = 768 16.3 / 21.9 (3, not taken), K = 2048 25.6 / 29.2 (4,
+// not taken), K = 4096 39.2 / 28.9 (8); M = 1021, N = 2043, K = 3072 34.2 /
+// 32.4 (4); M = 253, N = 507, K = 512 14.3 / 13.6 (2); with GELU M = 253, N =
+// 2043, K = 512 28.6 / 17.0 (2).
+constexpr PartPrice kLdsPrice{68, 320, 5, 160, 7, 2, 240};
+// Register-W GEMM (its parts summed by the last to arrive / by the launch):
 // 8-bit M = 100, K = 14336, N = 1000 55.2 / 20.8; 4-bit M = 128, K = 14336, N =
 // 4096 49.5 / 31.2; M = 80, K = 4096, N = 1000 24.1 / 14.5.
-inline int k_parts(int tiles, int KT, int most, bool halves, int step, const QmmArgs& a) {
+constexpr PartPrice kRwPrice{72, 400, 0, 240, 4, 4, 0};
+
+// K parts for a shape with few tiles (1: none, whole tiles or halves of a
+// split round) of KT steps, at most `most`: the cheapest.  Parts are whole
+// units of KT / most steps, so counts that do not divide them leave one part
+// longer than KT / S: priced at KT / S they took M = 330, K = 1024, N = 1778,
+// 6-bit as 3 parts of 1, 1 and 2 units, 19.6 us, against 18.2 as 4; M = 370, K
+// = 2048, N = 675, 6-bit 7 parts 20.1, 8 17.4; M = 75, K = 6144, N = 393, 3-bit
+// 20 parts 17.6, 24 15.0.
+inline int k_parts(int tiles, int KT, int most, bool halves, const PartPrice& c, const QmmArgs& a) {
     if (a.ws == nullptr || 2 * tiles > kCUs) return 1;
     const int cap = std::min(std::min(kCUs / tiles, most),
                              (int)((a.ws_bytes - split::kPartOffset) / ((size_t)tiles * kTileBytes)));
-    int best = 1, least = halves && a.epoch != 0u ? step * KT / 2 + 100 : step * KT;
+    int best = 1, least = halves && a.epoch != 0u ? c.step * KT / 2 + c.halves + c.halves_tile * tiles : c.step * KT;
+    if (a.has_epilogue()) least += c.fused;
     for (int S = 2; S <= cap; S++) {
-        const int cost = step * (KT / most) * ((most + S - 1) / S) + 60 + tiles * S;
+        const int parts = tiles * S, cost = c.step * (KT / most) * ((most + S - 1) / S) + c.launch +
+                                            c.part * std::min(parts, 128) + c.part_past * std::max(parts - 128, 0);
         if (cost < least) { least = cost; best = S; }
     }
     return best;

@@ -1097,8 +1097,8 @@ def test_group_gemm(ctx, oracle, bits, M, K, N, gs, sb, xd):
 @pytest.mark.parametrize("bits", [2, 3, 4, 5, 6])
 @pytest.mark.parametrize("M,K,N,gs,xd,sbd,od,act", [
     (70, 1536, 130, 64, F16, F16, F16, 3),     # 2 tiles, 6 parts of one window each, GELU
-    (257, 2816, 1003, 32, BF16, F16, BF16, 0),  # 16 tiles, 11 windows in uneven parts, odd N
-    (100, 768, 4096, 128, F16, BF16, F32, 2),  # 32 tiles, 3 parts, SiLU
+    (257, 2816, 1003, 32, BF16, F16, BF16, 0),  # 16 tiles, 11 windows in 6 parts of one or two, odd N
+    (100, 768, 2048, 128, F16, BF16, F32, 2),  # 16 tiles, 3 parts, SiLU
     (300, 11008, 4096, 64, BF16, BF16, F32, 0)])  # 64 tiles, 43 windows in 4 parts
 def test_lds_gemm_k_parts(ctx, oracle, bits, M, K, N, gs, xd, sbd, od, act):
     """The LDS-dequant GEMM in K parts summed by a second launch, with the
