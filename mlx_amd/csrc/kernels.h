@@ -93,8 +93,8 @@ size_t qgemm_sk_workspace(int M, int K, int N, int bits, int x_dtype, size_t cap
 // the same shape takes the same split, and the same result bits.  32 MiB of
 // partials: one 128 KiB tile of fp32 sums per CU (the K parts of the large
 // GEMMs; their split last round, at most 128 tiles of one K half each, and the
-// split-K small-M GEMM's largest split, 256 blocks of 32 KiB, need less).  The
-// first KiB holds tile counters and flags.
+// split-K small-M GEMM's largest split, 512 blocks of 32 KiB, need less).  The
+// first 4 KiB hold tile counters and flags (qsplit.h).
 constexpr size_t kSplitWorkspaceBytes = (32u << 20) + 4096;
 // MFMA GEMM for M > 64 with each wave's W operand dequantized in its own
 // registers: 4/8-bit codes, f16/bf16 x, K % 1024 == 0; NotSupported otherwise

@@ -24,9 +24,9 @@ extern template LuxStatus launch_bits<8>(const QmmArgs&, int, hipStream_t);
 // against 22.9).  So it runs unsplit from kUnsplitTiles tiles on, and split
 // only where the W-streaming kernel does not apply (K % 1024 != 0).
 constexpr int kUnsplitTiles = 192;
-// at most one block per CU; this also bounds the partials: 256 blocks x
-// 32 KiB = 8 MiB
-constexpr int kMaxBlocks = 256;
+// at most two blocks per CU; this also bounds the partials: 512 blocks x
+// 32 KiB = 16 MiB
+constexpr int kCUs = 256, kMaxBlocks = 512;
 
 bool applies(int M, int K, int N, int bits, int x_dtype) {
     if (M <= 8 || M > 64 || N <= 0 || (x_dtype != DT_F16 && x_dtype != DT_BF16) || K % kSS != 0) return false;
@@ -39,26 +39,35 @@ bool applies(int M, int K, int N, int bits, int x_dtype) {
     return (N + kCols - 1) / kCols >= kUnsplitTiles || K % 1024 != 0;
 }
 
-// the number of K parts S: 1 from kUnsplitTiles tiles on; else one block per
-// CU, but no more than sqrt(0.9 K / 128) parts (each adds a round trip of its
-// sums) of at least 2 super-steps, lowered until the workspace fits `cap`.
-// Parts need not be equal.  us per launch, against divisors of K / 128 that
-// gave at least kUnsplitTiles blocks: K = 11008 (86 super-steps: 2 parts, 64
-// blocks), N = 4096, 4-bit M = 16 / 32 / 64 31.5 / 32.8 / 44.8 -> 16.1 / 17.4 /
-// 23.7 (8 parts); K = 13440, N = 1000, 8-bit M = 64 39.7 -> 26; K = 3584, N =
-// 4096, 3-bit M = 64 (7 parts) 20.3 -> 18.8 (5); K = 2816, N = 8192, 8-bit M =
-// 20 14.7 -> 12.5 (4).  More blocks than CUs lose: K = 13824, N = 5120, M = 64
-// 29.2 (6 parts, 240 blocks) against 40.6 (7, 280).
+// the number of K parts S: 1 from kUnsplitTiles tiles on, else the cheapest
+// that leaves a part 2 super-steps and the workspace within `cap`.  In
+// hundredths of a us: 60 per super-step of the longest part (parts need not be
+// equal), more where CUs run two blocks (96 just past a block per CU, 126 at
+// two); for splitting at all 60; 40 (60 from 33 rows on) per trip of the last
+// part, which adds four at a time; and per part 10 and half (from 33 rows on,
+// all) of the tiles, which store and load together.  Fitted to 430 launches of
+// 1 to 180 tiles and 6 to 221 super-steps (0.8 % above the best split of each
+// in the mean).  us per launch (g64, f16, M = 12 / 48) with the cheapest divisor
+// of K / 128 that filled 192 blocks, with the square root of 0.9 K / 128 and at
+// most a block per CU, and with this: 4-bit K = 8448, N = 1019 17.5 / 27.6, 12.9
+// / 19.0, 12.3 / 18.5 (about 10 parts); K = 4608, N = 123 10.7 / 17.0, 11.2 /
+// 16.7, 9.9 / 14.8 (8); K = 28288, N = 251 17.6 / 26.9, 18.5 / 27.5, 16.6 / 25.5
+// (20); K = 2688, N = 7675 12.3 / 19.6, 10.5 / 16.8, 10.4 / 15.8 (4 and 3);
+// 2-bit K = 7040, N = 11387 24.5 / 32.7, 25.8 / 34.4, 24.4 / 34.4 (5 and 2); K =
+// 11008, N = 19195 54.8 / 70.3, 61.0 / 79.5, 42.4 / 54.8 (3).
 int choose_split(int M, int K, int N, size_t cap) {
     static_assert(kUnsplitTiles <= kMaxSplitTiles, "split tiles have counter slots");
     const int tiles = (N + kCols - 1) / kCols, steps = K / kSS;
     if (tiles >= kUnsplitTiles) return 1;
-    int S = std::min(steps / 2, kMaxBlocks / tiles);
-    while (S > 1 && (10 * S * S > 9 * steps || ws_bytes(S, M, N) > cap)) S--;
-    // two short parts save less than their meeting costs: three, or none (K =
-    // 896, N = 300, M = 33: 1 / 2 / 3 parts 9.7 / 10.5 / 9.4)
-    if (S == 2 && steps < 12) S = steps >= 6 && 3 * tiles <= kMaxBlocks && ws_bytes(3, M, N) <= cap ? 3 : 1;
-    return S < 1 ? 1 : S;
+    const int most = std::min(steps / 2, kMaxBlocks / tiles);
+    int best = 1, least = 60 * steps;
+    for (int S = 2; S <= most && ws_bytes(S, M, N) <= cap; S++) {
+        const int blocks = tiles * S, step = blocks > kCUs ? 66 + blocks * 30 / kCUs : 60;
+        const int cost = step * ((steps + S - 1) / S) + 60 + (M <= 32 ? 40 : 60) * ((S + 3) / 4) +
+                         (10 + (M <= 32 ? tiles / 2 : tiles)) * S;
+        if (cost < least) { least = cost; best = S; }
+    }
+    return best;
 }
 
 }  // namespace sk

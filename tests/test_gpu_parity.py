@@ -623,8 +623,8 @@ def test_small_gemm_two_tiles_parity(ctx, oracle, bits, xd, sbd, od):
 def test_split_k_gemm_parity(ctx, oracle, bits, xd, sbd, od):
     """8 < M <= 64 with K % 128 == 0 and K % 1024 != 0: the split-K small-M
     GEMM, the GEMM form ("dequantize to T, then matmul").  The shapes take
-    the K-part counts 1 (3 super-steps), 3 (of 9), 15 (of 30), 10 (of 20)
-    and 31 (of 62), one and two M tiles, ragged M and N; the parts meet
+    the K-part counts 1 (3 super-steps), 3 (of 9), 8 (of 30), 7 (of 20)
+    and 16 (of 62), one and two M tiles, ragged M and N; the parts meet
     through the context's workspace."""
     O = oracle
     for (M, K, N, gs) in [(9, 384, 77, 32), (12, 1152, 200, 64), (40, 3840, 300, 128),
@@ -650,12 +650,12 @@ def test_unsplit_wide_gemm_parity(ctx, oracle, M, xd, sbd, od):
 def test_split_k_shapes_in_sequence(ctx, oracle):
     """Split-K GEMM launches of different shapes back to back on one
     context workspace: a shape with few tiles and large partials (8 tiles,
-    14 K parts), then one with 188 tiles (2 K parts), then the first again.
+    7 K parts), then one with 125 tiles (2 K parts), then the first again.
     Every tile counter must read zero at the start of each launch, so no
     shape's partials may land on another's counter slots."""
     O = oracle
     A = (64, 3584, 1024, 4, 64)
-    B = (64, 2560, 24000, 4, 64)
+    B = (64, 2560, 16000, 4, 64)
     for i, (M, K, N, bits, gs) in enumerate([A, B, A]):
         x, w_q, s, b, _ = O.make_problem(M, K, N, bits, gs, BF16, BF16, seed=900 + N)
         y = run(ctx, x, w_q, s, b, M, K, N, gs, bits, BF16, BF16, F32, KERNELS["gemm"])
@@ -875,7 +875,7 @@ FUSED_CASES = [
     (6, 2048, 40, 8, 128, F16),     # mid-M ring kernel (8-bit)
     (32, 2048, 72, 4, 64, BF16),    # small-M GEMM
     (24, 1024, 8300, 3, 64, F16),   # small-M GEMM, two column tiles per block (N > 8192)
-    (40, 2560, 200, 4, 64, F16),    # split-K small-M GEMM (10 K parts)
+    (40, 2560, 200, 4, 64, F16),    # split-K small-M GEMM (7 K parts)
     (96, 512, 136, 4, 64, F16),     # large GEMM
     (3, 96, 20, 4, 32, F32),        # generic kernel (K % 64 != 0)
 ]
@@ -1137,8 +1137,9 @@ def test_lds_gemm_k_parts(ctx, oracle, bits, M, K, N, gs, xd, sbd, od, act):
 
 @pytest.mark.parametrize("bits", BITS)
 @pytest.mark.parametrize("M,K,N,gs,xd,sbd,od", [(33, 896, 300, 64, F16, F16, F32),   # 7 super-steps in 3 parts
-                                                (64, 11008, 260, 128, BF16, BF16, F32),  # 86 in 8
-                                                (12, 3200, 4097, 32, F16, F32, F16)])   # 25 in 4, one ragged tile
+                                                (64, 11008, 260, 128, BF16, BF16, F32),  # 86 in 15
+                                                (12, 3200, 4097, 32, F16, F32, F16),    # 25 in 7, one ragged tile
+                                                (12, 7040, 11300, 64, F16, F16, F32)])  # 55 in 5, two blocks per CU
 def test_split_k_gemm_uneven_parts(ctx, oracle, bits, M, K, N, gs, xd, sbd, od):
     """The split-K small-M GEMM with K parts of different lengths (fewer
     super-steps than the loads in flight among them), twice."""

@@ -22,7 +22,7 @@ pytestmark = pytest.mark.gpu
 
 # (M, K, N, bits, group size, x dtype, scales dtype, out dtype, kernel)
 CALLS = [
-    (64, 3584, 4096, 3, 64, F16, F16, F16, 0),     # split-K GEMM, 7 K parts, 224 blocks
+    (64, 3584, 4096, 3, 64, F16, F16, F16, 0),     # split-K GEMM, 4 K parts, 128 blocks
     (17, 1152, 200, 4, 32, BF16, BF16, F32, 2),    # split-K GEMM, 3 K parts, 6 blocks
     (512, 1024, 1024, 4, 64, BF16, BF16, F32, 2),  # large GEMM, 16 tiles, each in two K halves
     (300, 512, 200, 4, 64, F16, F16, F16, 2),      # large GEMM, 4 ragged tiles, each in two K halves
