@@ -1094,6 +1094,29 @@ def test_group_gemm(ctx, oracle, bits, M, K, N, gs, sb, xd):
     assert np.all(np.abs(y - want) <= (32 + K / 32 + 8) * 2.0**-24 * mag)
 
 
+@pytest.mark.parametrize("bits", [2, 4, 8])
+def test_group_gemm_many_parts_error(ctx, oracle, bits):
+    """56 K parts: their sum must not add much to the error of the parts.  A
+    rounding is off by 0.42 u of its result in the mean (u = 2^-24); adding P
+    equal parts one by one gives sqrt(P / 2) times that of the total, 2.2 u, in
+    fours and pairs sqrt(P / 8 + 2), 1.3 u.  With the 1.7 u of the parts
+    themselves (measured) that is 2.8 u and 2.1 u of the outputs' norm."""
+    from mlx_amd import runtime
+    O = oracle
+    M, K, N, gs = 16, 14336, 256, 64
+    assert ctx.kernel_name(M, K, N, gs, bits, F32, F32, F32) == "qgemm_grp_kernel"
+    x, w_q, s, b, _ = O.make_problem(M, K, N, bits, gs, F32, F32, seed=8900 + bits)
+    print(f"[case] group gemm 56 parts b{bits}", flush=True)
+    y = runtime.run_quantized_matmul(ctx, x, w_q, s, b, M, K, N, gs, bits, F32, F32, F32).astype(np.float64)
+    stream = np.unpackbits(w_q.view(np.uint8).reshape(N, -1), axis=1, bitorder="little")
+    q = (stream.reshape(N, K, bits) * (1 << np.arange(bits))).sum(-1).astype(np.float64)
+    w = np.repeat(s.astype(np.float64), gs, axis=1) * q + np.repeat(b.astype(np.float64), gs, axis=1)
+    want = x.astype(np.float64) @ w.T
+    err = float(np.linalg.norm(y - want) / np.linalg.norm(want))
+    print(f"group gemm 56 parts b{bits}: {err * 2**24:.2f} u")
+    assert err <= 2.4 * 2.0**-24
+
+
 @pytest.mark.parametrize("bits", [2, 3, 4, 5, 6])
 @pytest.mark.parametrize("M,K,N,gs,xd,sbd,od,act", [
     (70, 1536, 130, 64, F16, F16, F16, 3),     # 2 tiles, 6 parts of one window each, GELU
