@@ -8,8 +8,10 @@
 //  * a centred code (at most 8 bits) is a bf16 and an f16 number exactly;
 //  * 16-bit x goes in as it is; f32 x is the sum of three bf16 numbers
 //    exactly: its leading 8 significant bits, the next 8 and the last 8, each
-//    by truncation (so the first never rounds up to infinity; below 2^-109 the
-//    third underflows);
+//    by truncation (so the first never rounds up to infinity).  Below 2^-109
+//    the third underflows: a tile with a row of x that has nothing from 2^-100
+//    on is run once more, with such rows times 2^24 (watching for them costs 2 %
+//    of M = 64, K = N = 4096, 4-bit: 21.2 against 21.6 us);
 //  * a product of the two has at most 19 bits and is exact in the f32
 //    accumulator, which is started afresh for every group and then scaled
 //    into the f32 sums of y.
@@ -85,8 +87,10 @@ struct Lds {
     static constexpr int kScales = kCodes + 2 * BN * kCodeRow;
     static constexpr int kOut = BN + 4;                    // floats per row of the output tile
     static constexpr int kTile = BM * kOut * 4;            // two of them at the end (pairs of K parts)
+    static constexpr int kRows = 2 * kTile;                // past the tiles: 8 flags, then a value per row
+    static constexpr int kEnd = kRows + 32 + 4 * BM;
     static constexpr int kLoop = kScales + 2 * kWindow;
-    static constexpr int kBytes = kLoop > 2 * kTile ? kLoop : 2 * kTile;
+    static constexpr int kBytes = kLoop > kEnd ? kLoop : kEnd;
     static_assert(kBytes <= 160 * 1024, "LDS");
 };
 
@@ -137,13 +141,22 @@ __device__ __forceinline__ u4 codes8(const uint32_t* w, int j) {
     return r;
 }
 
-// BITS: code width; TX: type of x; SBF: f32 scales (else 16-bit ones, sb_dt says which); MT:
-// 32-row tiles
+// a thread's 16-byte vectors of the output tile: 4 columns of rows tid / 32 + 16 i
+template <int MT>
+constexpr int kOutVecs = 32 * MT * BN / 4 / kThreads;
+// rows of f32 x whose third terms have underflowed, and what such x is taken times
+constexpr float kSmall = 0x1p-100f, kSmallUp = 0x1p24f, kSmallDown = 0x1p-24f;
+
+// One run over steps s0 .. s1 - 1 of the tile at (m0, n0): its sums in o.
+// BITS: code width; TX: type of x; SBF: f32 scales (else 16-bit ones, sb_dt
+// says which); MT: 32-row tiles.  f32 x: true where a row has nothing from
+// kSmall on; again then takes such rows times kSmallUp (bit i of small: the
+// thread's load i of x is of one, of rows: its vector i of the output).
 template <int BITS, int TX, bool SBF, int MT>
-__global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
-    const void* __restrict__ x, const uint32_t* __restrict__ wq, const void* __restrict__ scales,
-    const void* __restrict__ biases, void* __restrict__ y, int M, int K, int N, int gshift, int sb_dt, Epilogue ep,
-    int mtiles, int tiles, int parts, void* __restrict__ ws) {
+__device__ __forceinline__ bool run_tile(uint8_t* lds, const void* __restrict__ x, const uint32_t* __restrict__ wq,
+                                         const void* __restrict__ scales, const void* __restrict__ biases, int M, int K,
+                                         int N, int gshift, int sb_dt, int m0, int n0, int s0, int s1, bool again,
+                                         uint32_t& small, uint32_t& rows, f4 (&o)[kOutVecs<MT>]) {
     constexpr int P = TX == DT_F32 ? 3 : 1;       // planes of x
     using L = Lds<MT, BITS, P>;
     constexpr int BM = L::BM, NT = 2;
@@ -155,15 +168,14 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
     constexpr int XR = kThreads / XC;             // rows per pass of x loads
     constexpr int kSb = SBF ? 4 : 2;
     constexpr float C = (float)(1 << (BITS - 1));
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    const int tid = threadIdx.x, lane = tid & 63;
+    int tid = threadIdx.x;
+    // (addresses of a run are its own: kept over both they cost 80 registers)
+    if constexpr (TX == DT_F32) asm volatile("" : "+v"(tid));
+    const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kg = wave >> 1, nw = wave & 1;
     const int c = lane & 31, h = lane >> 5;
-    const int tile = (int)blockIdx.x % tiles, part = (int)blockIdx.x / tiles;
-    const int m0 = tile % mtiles * BM, n0 = tile / mtiles * BN;
     const int steps = (K + BK - 1) / BK;
-    const int s0 = (int)((long long)steps * part / parts), s1 = (int)((long long)steps * (part + 1) / parts);
 
     // x: thread t loads 16 bytes (chunk t % XC) of rows t / XC, + XR, ...; rows
     // past M re-read the last (never stored), k past K are zeros
@@ -215,8 +227,9 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
             if (BITS % 4 == 0 || tid + kThreads * i < BN * BITS) *reinterpret_cast<u4*>(d + cd[i]) = o.c[i];
     };
     // load i of step s into the planes of stage st; the sum over the thread's
-    // XE k.  fix: an infinity's residue (inf - inf) is 0; a NaN's stays NaN
-    auto split = [&](const Raw& o, int s, int i, uint8_t* st, float& big, auto fix) LXQ_INLINE {
+    // XE k.  fix: an infinity's residue (inf - inf) is 0; a NaN's stays NaN.
+    // low: the third terms' bits, of which the last 16 are what it has lost
+    auto split = [&](const Raw& o, int s, int i, uint8_t* st, uint32_t& low, auto fix) LXQ_INLINE {
         u4 v = o.x[i];
         if ((s + 1) * BK > K && s * BK + XE * xc >= K) v = u4{0u, 0u, 0u, 0u};
         const int row = xr + XR * i;
@@ -228,12 +241,12 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 f[e] = __uint_as_float(v[e]);
-                big = fmaxf(big, fabsf(f[e]));
                 p[0][e] = v[e] & 0xffff0000u;
                 float r = f[e] - __uint_as_float(p[0][e]);
                 if constexpr (decltype(fix)::value) r = __builtin_isinf(f[e]) ? 0.f : r;
                 p[1][e] = __float_as_uint(r) & 0xffff0000u;
                 p[2][e] = __float_as_uint(r - __uint_as_float(p[1][e]));
+                low |= p[2][e];
             }
 #pragma unroll
             for (int q = 0; q < 3; q++)
@@ -250,12 +263,12 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
             return (f[0] + f[1]) + (f[2] + f[3]);
         }
     };
-    // after the splits of a step: the rare step that holds an infinity is
-    // split again; the sums over 32 k (32 / XE lanes)
-    auto finish = [&](const Raw& o, int s, float (&sum)[XL], uint8_t* st, float big) LXQ_INLINE {
-        if (TX == DT_F32 && __any(big == __builtin_inff())) {
+    // after the splits of a step: the rare step that may hold an infinity (its
+    // third term is a NaN) is split again; the sums over 32 k (32 / XE lanes)
+    auto finish = [&](const Raw& o, int s, float (&sum)[XL], uint8_t* st, uint32_t low) LXQ_INLINE {
+        if (TX == DT_F32 && __any((low & 0x7f800000u) == 0x7f800000u)) {
 #pragma unroll
-            for (int i = 0; i < XL; i++) split(o, s, i, st, big, std::true_type{});
+            for (int i = 0; i < XL; i++) split(o, s, i, st, low, std::true_type{});
         }
 #pragma unroll
         for (int i = 0; i < XL; i++) sum[i] += dpp_f<0xB1>(sum[i]);
@@ -278,6 +291,15 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
         return sb_dt == DT_F16 ? f16_to_f32(raw) : bf16_to_f32(raw);
     };
 
+    auto scale_x = [&](Raw& o) LXQ_INLINE {
+#pragma unroll
+        for (int i = 0; i < XL; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if ((small >> i) & 1u) o.x[i][e] = __float_as_uint(__uint_as_float(o.x[i][e]) * kSmallUp);
+    };
+    uint32_t lost = 0;  // the third terms' bits of all steps
+
     f32x16 acc[MT][NT];
 #pragma unroll
     for (int i = 0; i < MT; i++)
@@ -290,6 +312,7 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
     // step s from stage (s - s0) % 2; o holds step s + 1 as loaded (past the
     // last step: the last again, into a stage that nobody reads)
     auto step = [&](int s, Raw& o) LXQ_INLINE {
+        if (TX == DT_F32 && again) scale_x(o);
         const int stage = (s - s0) & 1, sn = min(s + 1, s1 - 1);
         const uint8_t* st = lds + stage * L::kStage;
         uint8_t* other = lds + (stage ^ 1) * L::kStage;
@@ -321,7 +344,8 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
             bi[t] = in ? fmaf(sc[t], C, sb_f(ss + BN * L::kScaleRow)) : 0.f;
         }
         store_codes(o, stage ^ 1);
-        float sum[XL], big = 0.f;
+        float sum[XL];
+        uint32_t low = 0;
         f32x16 g[MT][NT];
 #pragma unroll
         for (int j = 0; j < 2; j++) {
@@ -352,9 +376,10 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
                         }
                     }
 #pragma unroll
-            for (int i = j * XL / 2; i < (j + 1) * XL / 2; i++) sum[i] = split(o, sn, i, other, big, std::false_type{});
+            for (int i = j * XL / 2; i < (j + 1) * XL / 2; i++) sum[i] = split(o, sn, i, other, low, std::false_type{});
         }
-        finish(o, sn, sum, other, big);
+        finish(o, sn, sum, other, low);
+        lost |= low;
         load(o, min(s + 2, s1 - 1));
         const uint8_t* sums = st + L::kSums + kg * (BM * 4);
 #pragma unroll
@@ -376,12 +401,15 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
 
     Raw next;
     {
-        float sum[XL], big = 0.f;
+        float sum[XL];
+        uint32_t low = 0;
         load(next, s0);
         const u4 w0 = load_win(s0 >> gws);
+        if (TX == DT_F32 && again) scale_x(next);
 #pragma unroll
-        for (int i = 0; i < XL; i++) sum[i] = split(next, s0, i, lds, big, std::false_type{});
-        finish(next, s0, sum, lds, big);
+        for (int i = 0; i < XL; i++) sum[i] = split(next, s0, i, lds, low, std::false_type{});
+        finish(next, s0, sum, lds, low);
+        lost |= low;
         store_codes(next, 0);
         load(next, min(s0 + 1, s1 - 1));
         store_win(s0 >> gws, w0);
@@ -393,6 +421,11 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
     // 32 x 32 tile, register v its row 8 (v / 4) + 4 h + v % 4): parts 0 and 2
     // store, 1 and 3 add theirs
     float* ot = reinterpret_cast<float*>(lds + (kg >> 1) * L::kTile);
+    uint32_t* flags = reinterpret_cast<uint32_t*>(lds + L::kRows);
+    if constexpr (TX == DT_F32) {
+        const bool any = __any((lost & 0xffffu) != 0u);
+        if (lane == 0) flags[wave] = any ? 1u : 0u;
+    }
 #pragma unroll
     for (int half = 0; half < 2; half++) {
         if ((kg & 1) == half) {
@@ -408,16 +441,65 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
         }
         __syncthreads();
     }
-    // thread: 4 columns (16 bytes) of rows tid / 32 + 16 i
     const int oc = 4 * (tid & 31), orow = tid >> 5;
-    constexpr int kVec = BM * BN / 4 / kThreads;
-    constexpr uint32_t kSlot = BM * BN * 4;
-    f4 o[kVec];
 #pragma unroll
-    for (int i = 0; i < kVec; i++) {
+    for (int i = 0; i < kOutVecs<MT>; i++) {
         const float* d = reinterpret_cast<const float*>(lds) + (orow + 16 * i) * L::kOut + oc;
         o[i] = *reinterpret_cast<const f4*>(d) + *reinterpret_cast<const f4*>(d + L::kTile / 4);
+        if (TX == DT_F32 && again && ((rows >> i) & 1u)) o[i] *= kSmallDown;
     }
+    if constexpr (TX != DT_F32) return false;
+    if (again) return false;
+    const u4 f0 = *reinterpret_cast<const u4*>(flags), f1 = *reinterpret_cast<const u4*>(flags + 4), fa = f0 | f1;
+    if ((fa[0] | fa[1] | fa[2] | fa[3]) == 0u) return false;
+    // bits were lost somewhere (a tail of SiLU or of an exponential will do
+    // it): the largest x of each row
+    float most[XL];
+#pragma unroll
+    for (int i = 0; i < XL; i++) most[i] = 0.f;
+    for (int s = s0; s < s1; s++) {
+        load(next, s);
+#pragma unroll
+        for (int i = 0; i < XL; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) most[i] = fmaxf(most[i], fabsf(__uint_as_float(next.x[i][e])));
+    }
+    float* row_most = reinterpret_cast<float*>(flags + 8);
+#pragma unroll
+    for (int i = 0; i < XL; i++) {
+#pragma unroll
+        for (int d = 1; d < XC; d <<= 1) most[i] = fmaxf(most[i], __shfl_xor(most[i], d));
+        if (xc == 0) row_most[xr + XR * i] = most[i];
+        if (most[i] < kSmall) small |= 1u << i;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kOutVecs<MT>; i++)
+        if (row_most[orow + 16 * i] < kSmall) rows |= 1u << i;
+    const float r = row_most[lane & (BM - 1)];
+    __syncthreads();  // the tiles and the rows are read before another run's stages
+    return __any(r > 0.f && r < kSmall);
+}
+
+template <int BITS, int TX, bool SBF, int MT>
+__global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
+    const void* __restrict__ x, const uint32_t* __restrict__ wq, const void* __restrict__ scales,
+    const void* __restrict__ biases, void* __restrict__ y, int M, int K, int N, int gshift, int sb_dt, Epilogue ep,
+    int mtiles, int tiles, int parts, void* __restrict__ ws) {
+    constexpr int BM = 32 * MT, kVec = kOutVecs<MT>;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int tile = (int)blockIdx.x % tiles, part = (int)blockIdx.x / tiles;
+    const int m0 = tile % mtiles * BM, n0 = tile / mtiles * BN;
+    const int steps = (K + BK - 1) / BK;
+    const int s0 = (int)((long long)steps * part / parts), s1 = (int)((long long)steps * (part + 1) / parts);
+    f4 o[kVec];
+    uint32_t small = 0, rows = 0;
+    bool again = false;
+    while (run_tile<BITS, TX, SBF, MT>(lds, x, wq, scales, biases, M, K, N, gshift, sb_dt, m0, n0, s0, s1, again, small,
+                                       rows, o))
+        again = true;
+    const int tid = threadIdx.x, oc = 4 * (tid & 31), orow = tid >> 5;
+    constexpr uint32_t kSlot = BM * BN * 4;
     if (parts > 1) {
         const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(
             static_cast<uint8_t*>(ws) + split::kPartOffset, 0, (int)((uint32_t)(tiles * parts) * kSlot), 0x00020000);

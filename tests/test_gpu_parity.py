@@ -1177,24 +1177,68 @@ def test_split_k_gemm_uneven_parts(ctx, oracle, bits, M, K, N, gs, xd, sbd, od):
     check_output(O, np.ascontiguousarray(ys[0][rows]), want, od, f"uneven parts b{bits} M{M} K{K} N{N}")
 
 
+def _exact_rows(O, x, w_q, s, b, bits, gs):
+    """(float64 product, bound on an f32 output's error: (32 + K / 32 + 8) 2^-24
+    of the sum of its terms' magnitudes) for f32 x, scales and biases."""
+    N, K = w_q.shape[0], x.shape[1]
+    stream = np.unpackbits(w_q.view(np.uint8).reshape(N, -1), axis=1, bitorder="little")
+    q = (stream.reshape(N, K, bits) * (1 << np.arange(bits))).sum(-1).astype(np.float64)
+    sf, bf = (np.repeat(t.astype(np.float64), gs, axis=1) for t in (s, b))
+    c = 2.0 ** (bits - 1)
+    xf = x.astype(np.float64)
+    mag = np.abs(xf) @ (sf * np.abs(q - c) + np.abs(bf + c * sf)).T
+    return xf @ (sf * q + bf).T, (32 + K / 32 + 8) * 2.0**-24 * mag
+
+
 def test_f32_gemm_special_values(ctx, oracle):
     """An infinity or a NaN in a row of x reaches that row's outputs and no
-    other, and x of 2^120, all mantissa bits set, stays finite in its three
-    terms (times an 8-bit code it is just below the f32 range)."""
+    other, and x just below 2^120, all mantissa bits set, keeps its three terms
+    (times a centred 8-bit code it is just below the f32 range)."""
     from mlx_amd import runtime
     O = oracle
     M, K, N = 20, 256, 130
-    x, w_q, s, b, _ = O.make_problem(M, K, N, 4, 64, F32, F32, seed=3)
-    clean = runtime.run_quantized_matmul(ctx, x, w_q, s, b, M, K, N, 64, 4, F32, F32, F32)
+    assert ctx.kernel_name(M, K, N, 64, 8, F32, F32, F32) == "qgemm_grp_kernel"
+    x, w_q, s, b, _ = O.make_problem(M, K, N, 8, 64, F32, F32, seed=3)
+    clean = runtime.run_quantized_matmul(ctx, x, w_q, s, b, M, K, N, 64, 8, F32, F32, F32)
     z = x.copy()
     z[2, 5], z[7, 200], z[9, 0] = np.inf, np.nan, -np.inf
-    z[11, 77] = np.finfo(np.float32).max / 256
+    z[11, 77] = np.nextafter(np.float32(2.0**120), np.float32(0))
     print("[case] f32 gemm special values", flush=True)
-    y = runtime.run_quantized_matmul(ctx, z, w_q, s, b, M, K, N, 64, 4, F32, F32, F32)
+    y = runtime.run_quantized_matmul(ctx, z, w_q, s, b, M, K, N, 64, 8, F32, F32, F32)
     for m in (2, 7, 9):
         assert not np.isfinite(y[m]).any()
+    want, bound = _exact_rows(O, z[11:12], w_q, s, b, 8, 64)
     assert np.isfinite(y[11]).all()
+    assert np.all(np.abs(y[11:12] - want) <= bound)
     rest = [m for m in range(M) if m not in (2, 7, 9, 11)]
+    assert np.array_equal(y[rest], clean[rest])
+
+
+@pytest.mark.parametrize("M,K,N,bits,gs", [(24, 192, 130, 4, 64),    # one part, a last half step
+                                           (64, 4160, 300, 3, 32),   # K parts, two 32-row tiles
+                                           (70, 1024, 129, 8, 128)])
+def test_f32_gemm_small_x(ctx, oracle, M, K, N, bits, gs):
+    """Rows of x down to f32's smallest numbers, where the last of the three
+    bf16 terms underflows: each is as exact as a row of ordinary size, beside
+    rows of zeros, of ordinary x, and of ordinary x with such numbers among
+    them.  (Scales of 2^30 keep the outputs normal.)"""
+    from mlx_amd import runtime
+    O = oracle
+    assert ctx.kernel_name(M, K, N, gs, bits, F32, F32, F32) == "qgemm_grp_kernel"
+    x, w_q, s, b, _ = O.make_problem(M, K, N, bits, gs, F32, F32, seed=8950 + bits)
+    s, b = (np.ldexp(t, 30).astype(np.float32) for t in (s, b))
+    clean = runtime.run_quantized_matmul(ctx, x, w_q, s, b, M, K, N, gs, bits, F32, F32, F32)
+    z = x.copy()
+    for m, e in enumerate((-98, -104, -110, -114, -118, -122, -126, -131, -137, -143)):
+        z[2 * m] = np.ldexp(x[2 * m], e)
+    z[1] = 0.0
+    z[3, ::2] = np.ldexp(x[3, ::2], -125)
+    z[M - 1, : K // 2] = np.ldexp(x[M - 1, : K // 2], -112)
+    print(f"[case] f32 gemm small x M={M} K={K} N={N} b{bits}", flush=True)
+    y = runtime.run_quantized_matmul(ctx, z, w_q, s, b, M, K, N, gs, bits, F32, F32, F32)
+    want, bound = _exact_rows(O, z, w_q, s, b, bits, gs)
+    assert np.all(np.abs(y - want) <= bound)
+    rest = [m for m in range(5, M - 1) if m >= 20 or m % 2]
     assert np.array_equal(y[rest], clean[rest])
 
 
