@@ -206,12 +206,18 @@ __attribute__((visibility("default"))) bool lux_gpu_backend_quant_init(const lux
  * allocation needs 256 bytes left after it).  `stream` is a hipStream_t of
  * that device (NULL: the null stream).  Same kernels, selection, results and shape and
  * dtype errors as op_quantized_matmul_ex.  The partial sums, tile counters
- * and flags of the split-K small-M GEMM and of the large GEMM's split last
- * round live in a 32 MiB (+ 4 KiB) static device array that
- * each GPU holds until the process ends (shapes whose split would need more
- * are INVALID_ARGUMENT; the split rule keeps every shape within it).  All
- * calls on one GPU share that array: calls that overlap in time on one GPU
- * (concurrent streams, or threads) race and give wrong results.  The first
+ * and flags of the kernels that split K live in a 32 MiB (+ 4 KiB) static
+ * device array that each GPU holds until the process ends (shapes whose split
+ * would need more are INVALID_ARGUMENT; the split rule keeps every shape
+ * within it): the split-K small-M GEMM, the large GEMMs' K parts and split
+ * last round, and the group-wise GEMM, which also takes GEMV requests -- f32 x
+ * from 9 rows on (from 5 at widths or K the 4-row kernel does not take), and
+ * 16-bit x from 4 rows on at shapes no other multi-row kernel takes.  All
+ * calls on one GPU share that array, whichever kernel they run: calls that
+ * overlap in time on one GPU (concurrent streams or threads, or a replayed
+ * graph beside another call) race and give wrong results, and may leave a
+ * counter that makes later calls wrong too.  A caller with several streams
+ * must order its calls on one GPU, or give each stream a context.  The first
  * call on a device clears the array with a kernel on its stream, so that
  * call must not be made under stream capture: it returns NOT_SUPPORTED
  * there (make one eager call on the device first; later calls may be

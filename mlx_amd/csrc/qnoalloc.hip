@@ -4,12 +4,14 @@
 // caller-owned device pointers and a caller stream, with no context: it
 // calls no allocating routine, for callers that cannot (code under graph
 // capture, serving loops that forbid allocation).  The kernels that need
-// device memory beyond their operands -- the split-K small-M GEMM and the
-// large GEMM's split last round (partial sums, tile counters and flags) --
-// take it from `scratch` below: a static device array that each GPU holds
-// from module load until the process ends.  Its size is the context
-// workspace's, so a shape takes the same K split, and gives the same bits,
-// on both entry points.
+// device memory beyond their operands -- partial sums, tile counters and flags
+// of the split-K small-M GEMM, the group-wise GEMM's and the large GEMMs' K
+// parts and the latter's split last round -- take it from `scratch` below: a
+// static device array that each GPU holds from module load until the process
+// ends.  Its size is the context workspace's, so a shape takes the same K
+// split, and gives the same bits, on both entry points.  Calls on one GPU must
+// not overlap: two that do share partial sums and counters, and a count that
+// falls between another launch's last count and its reset stays in the array.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -36,7 +38,7 @@ __global__ void clear_words(uint32_t* p, size_t n) {
 
 // once per device, with that device current: look up the array's device
 // address and clear it (a kernel on `st`, ordered before this call's work;
-// the GEMMs return their counters and flags to zero after every launch).
+// the kernels return their counters and flags to rest after every launch).
 // That first call must not be under stream capture: the clear would become
 // a node of the caller's graph and run on every replay, after later calls
 // have relied on the array being clear once.  It is refused instead.
