@@ -538,14 +538,13 @@ __device__ __forceinline__ void setup_ctx(Ctx<C>& t, const Unit& w, uint8_t* lds
     for (int tt = 0; tt < 2; tt++) t.sb_lds[tt] = wave * C::WN * 32 + (32 * tt + c) * 16;
 }
 
-// rows [32 I0, 32 I1) of the block's tile, through the output stage, in
-// 16-bit type TO into LDS at dst (row stride rs bytes, row 32 I0 first):
+// rows [32 I0, 32 I1) of the block's tile, in 16-bit type TO into LDS at dst (row stride rs bytes, row 32 I0 first):
 // lane (c, h) holds column c and rows 8 (v / 4) + 4 h + v % 4 of each 32 x
 // 32 tile, so VGPRs v and v + 1 are two rows of one column, converted
 // together
-template <class C, bool EPI, int TO, int I0 = 0, int I1 = C::MT>
-__device__ __forceinline__ void stage16(uint8_t* dst, int rs, const f32x16 (&acc)[C::MT][C::NT], const Epilogue& ep,
-                                        int n0, int N, int wave, int c, int h) {
+template <class C, int TO, int I0 = 0, int I1 = C::MT>
+__device__ __forceinline__ void stage16(uint8_t* dst, int rs, const f32x16 (&acc)[C::MT][C::NT], int wave, int c,
+                                        int h) {
 #pragma unroll
     for (int i = I0; i < I1; i++)
 #pragma unroll
@@ -554,14 +553,7 @@ __device__ __forceinline__ void stage16(uint8_t* dst, int rs, const f32x16 (&acc
 #pragma unroll
             for (int v = 0; v < 16; v += 2) {
                 const int ml = 32 * (i - I0) + 8 * (v >> 2) + 4 * h + (v & 3);
-                float o0 = acc[i][tt][v], o1 = acc[i][tt][v + 1];
-                if constexpr (EPI) {
-                    if (n0 + nl < N) {
-                        o0 = apply_epilogue(ep, (size_t)(n0 + nl), o0);
-                        o1 = apply_epilogue(ep, (size_t)(n0 + nl), o1);
-                    }
-                }
-                const uint32_t pk = pack2<TO>(o0, o1);
+                const uint32_t pk = pack2<TO>(acc[i][tt][v], acc[i][tt][v + 1]);
                 uint8_t* d = dst + ml * rs + nl * 2;
                 *reinterpret_cast<uint16_t*>(d) = (uint16_t)pk;
                 *reinterpret_cast<uint16_t*>(d + rs) = (uint16_t)(pk >> 16);
@@ -584,13 +576,13 @@ constexpr bool kStageAbove = C::kLds + kHandLds<C> <= 160 * 1024;
 
 // half P of a handed-over tile (rows P BM / 2 ..+BM / 2) staged at hs and
 // read back as the thread's chunks P kHand / 2 ..
-template <class C, bool EPI, int P>
-__device__ __forceinline__ void hand_half(uint8_t* hs, int rs, const f32x16 (&acc)[C::MT][C::NT], const Epilogue& ep,
-                                          int n0, int N, int wave, int c, int h, int tid, u4 (&val)[kHand<C>]) {
+template <class C, int P>
+__device__ __forceinline__ void hand_half(uint8_t* hs, int rs, const f32x16 (&acc)[C::MT][C::NT], int out_dt, int wave,
+                                          int c, int h, int tid, u4 (&val)[kHand<C>]) {
     static_assert(C::MT % 2 == 0 && kHand<C> % 2 == 0, "halves of whole 32-row tiles and chunk rounds");
     constexpr int I0 = P * C::MT / 2, I1 = I0 + C::MT / 2, kHalf = kHand<C> / 2;
-    if (ep.out_dt == DT_BF16) stage16<C, EPI, DT_BF16, I0, I1>(hs, rs, acc, ep, n0, N, wave, c, h);
-    else stage16<C, EPI, DT_F16, I0, I1>(hs, rs, acc, ep, n0, N, wave, c, h);
+    if (out_dt == DT_BF16) stage16<C, DT_BF16, I0, I1>(hs, rs, acc, wave, c, h);
+    else stage16<C, DT_F16, I0, I1>(hs, rs, acc, wave, c, h);
     barrier_lds();
 #pragma unroll
     for (int i = 0; i < kHalf; i++) {
@@ -687,13 +679,13 @@ __global__ __launch_bounds__(C::kThreads, 1) void qgemm_rw_kernel(
             // rings in two passes of BM / 2 rows
             next_unit(un);
             uint8_t* hs = lds + C::kLds;
-            hand_half<C, EPI, 0>(hs, rs, acc, ep, no, N, wave, c, h, tid, val);
+            hand_half<C, 0>(hs, rs, acc, ep.out_dt, wave, c, h, tid, val);
             barrier_lds();  // half 0 is read before half 1 overwrites it
-            hand_half<C, EPI, 1>(hs, rs, acc, ep, no, N, wave, c, h, tid, val);
+            hand_half<C, 1>(hs, rs, acc, ep.out_dt, wave, c, h, tid, val);
         } else {
             // the tile in the rings in one pass, then the next unit's transfers
-            if (ep.out_dt == DT_BF16) stage16<C, EPI, DT_BF16>(lds, rs, acc, ep, no, N, wave, c, h);
-            else stage16<C, EPI, DT_F16>(lds, rs, acc, ep, no, N, wave, c, h);
+            if (ep.out_dt == DT_BF16) stage16<C, DT_BF16>(lds, rs, acc, wave, c, h);
+            else stage16<C, DT_F16>(lds, rs, acc, wave, c, h);
             barrier_lds();
 #pragma unroll
             for (int i = 0; i < kHand<C>; i++) {
@@ -780,8 +772,8 @@ __global__ __launch_bounds__(C::kThreads, 1) void qgemm_rw_kernel(
         // vector stores need 16-byte aligned rows: N a multiple of 8, y aligned
         const bool vec = (((uintptr_t)y) & 15) == 0 && N % 8 == 0;
         barrier();
-        if (ep.out_dt == DT_BF16) stage16<C, EPI, DT_BF16>(lds, rs, acc, ep, n0, N, wave, c, h);
-        else stage16<C, EPI, DT_F16>(lds, rs, acc, ep, n0, N, wave, c, h);
+        if (ep.out_dt == DT_BF16) stage16<C, DT_BF16>(lds, rs, acc, wave, c, h);
+        else stage16<C, DT_F16>(lds, rs, acc, wave, c, h);
         barrier_lds();
         // row r: BN * 2 bytes = 32 16-byte chunks
         for (int q = tid; q < BM * 32; q += C::kThreads) {

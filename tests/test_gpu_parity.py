@@ -829,8 +829,8 @@ def test_rw_gemm_persistent_parity(ctx, oracle, case):
     unit's first transfers land.  Whole outputs against the oracle's
     dequantize-to-T form: ragged M (the last M tile's rows past M are
     dropped by offset), ragged N (N % 256 != 0), the hand-over into a split
-    K half, both 16-bit outputs, and the fused output stage (bias and
-    activation applied in the hand-over's staging)."""
+    K half and both 16-bit outputs.  The fused output stage takes no part in
+    the hand-over: with it a block runs one unit and stores it row by row."""
     from mlx_amd import runtime
     O = oracle
     M, K, N, bits, gs, xd, sbd = case
