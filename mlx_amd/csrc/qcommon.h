@@ -31,6 +31,17 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float v) {
     return __builtin_bit_cast(uint16_t, (__bf16)v);
 }
 
+// two fp32 values -> a packed pair of T, RNE, as one packed conversion: a
+// scalar (_Float16) cast of an fmaf result lets the compiler fuse both into
+// v_fma_mixlo_f16, which rounds once (exact -> f16) where the format rounds
+// twice (exact -> fp32 -> f16) and differs at f16 ties
+template <int T>
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    if constexpr (T == DT_BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, bf16x2));
+    else return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, f16x2));
+}
+
 // value of v after a round trip through dtype dt
 __device__ __forceinline__ float round_dt(float v, int dt) {
     if (dt == DT_F32) return v;

@@ -33,17 +33,6 @@ __device__ __forceinline__ float sb_at(const void* p, size_t i) {
     else return bf16_to_f32(static_cast<const uint16_t*>(p)[i]);
 }
 
-// two fp32 values -> a packed pair of T, RNE (a scalar f16 cast of an fmaf
-// result could fuse into one rounding where the format rounds twice)
-template <int T>
-__device__ __forceinline__ uint32_t cvt_pk(float a, float b) {
-    typedef float f2 __attribute__((ext_vector_type(2)));
-    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    if constexpr (T == DT_BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, b2));
-    else return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, h2));
-}
-
 template <int BITS, int SB, int OT, int U>
 __global__ __launch_bounds__(256) void dequant_kernel(const uint32_t* __restrict__ wq, const void* __restrict__ sc,
                                                       const void* __restrict__ bi, void* __restrict__ out,
@@ -96,7 +85,7 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint32_t* __restrict
             typedef float f4 __attribute__((ext_vector_type(4)));
             *o = __builtin_bit_cast(o4, f4{v[0], v[1], v[2], v[3]});
         } else {
-            *o = o4{cvt_pk<OT>(v[0], v[1]), cvt_pk<OT>(v[2], v[3]), cvt_pk<OT>(v[4], v[5]), cvt_pk<OT>(v[6], v[7])};
+            *o = o4{pack2<OT>(v[0], v[1]), pack2<OT>(v[2], v[3]), pack2<OT>(v[4], v[5]), pack2<OT>(v[6], v[7])};
         }
     }
 }

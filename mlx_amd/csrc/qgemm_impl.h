@@ -78,18 +78,6 @@ static_assert(kCUs / 2 <= split::kMaxHalfTiles, "split tiles within the workspac
 // r and r + 8 get different permutations)
 __device__ __forceinline__ int swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
-// two fp32 values -> packed pair of T, RNE (one v_cvt_pk_{bf16,f16}_f32)
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-template <int TX>
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-    if constexpr (TX == DT_BF16)
-        return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2_t));
-    else
-        return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), f16x2_t));
-}
-
 // 8 codes (8c .. 8c+7) of a 32-code half unit held in BITS words, as fp32.
 // 4-bit and 8-bit codes are spread to bytes for v_cvt_f32_ubyte{0..3};
 // other widths extract each code with a bitfield op.

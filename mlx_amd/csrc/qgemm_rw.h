@@ -165,20 +165,6 @@ __device__ __forceinline__ f32x16 mfma(const u4& a, const u4& b, const f32x16& c
                                                      0, 0, 0);
 }
 
-// two fp32 values -> a packed pair of T, RNE, one packed conversion (a
-// scalar f16 cast of an fmaf result would fuse into v_fma_mixlo_f16, which
-// rounds once where the format rounds twice)
-template <int TX>
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-    typedef float f2 __attribute__((ext_vector_type(2)));
-    if constexpr (TX == DT_BF16) {
-        typedef __bf16 t2 __attribute__((ext_vector_type(2)));
-        return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, t2));
-    } else {
-        typedef _Float16 t2 __attribute__((ext_vector_type(2)));
-        return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, t2));
-    }
-}
 __device__ __forceinline__ float lo(uint32_t m) { return (float)__builtin_bit_cast(h2, m)[0]; }
 __device__ __forceinline__ float hi(uint32_t m) { return (float)__builtin_bit_cast(h2, m)[1]; }
 

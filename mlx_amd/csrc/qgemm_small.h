@@ -65,22 +65,6 @@ __device__ __forceinline__ float sb_val(uint32_t w) {
     else if constexpr (SB == DT_F16) return f16_to_f32(w & 0xffffu);
     else return bf16_to_f32(w & 0xffffu);
 }
-// two fp32 values -> a packed pair of T, RNE, as one packed conversion: a
-// scalar (_Float16) cast of an fmaf result lets the compiler fuse both into
-// v_fma_mixlo_f16, which rounds once (exact -> f16) where the format rounds
-// twice (exact -> fp32 -> f16) and differs at f16 ties
-template <int TX>
-__device__ __forceinline__ uint32_t pack_t(float a, float b) {
-    typedef float f2 __attribute__((ext_vector_type(2)));
-    if constexpr (TX == DT_BF16) {
-        typedef __bf16 t2 __attribute__((ext_vector_type(2)));
-        return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, t2));
-    } else {
-        typedef _Float16 t2 __attribute__((ext_vector_type(2)));
-        return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, t2));
-    }
-}
-
 // the f16 in the low / high half of a word, as fp32 (v_fma_mix_f32 reads it
 // in place when the product feeds an FMA)
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
@@ -174,10 +158,10 @@ __device__ __forceinline__ u4 w_operand(const uint32_t* c, float sc, float bi, i
         for (int e = 0; e < 8; e++) q[e] = fmaf(sc, (float)unit_code<BITS>(c, 8 * s + e), bi);
     }
     u4 r;
-    r.x = pack_t<TX>(q[0], q[1]);
-    r.y = pack_t<TX>(q[2], q[3]);
-    r.z = pack_t<TX>(q[4], q[5]);
-    r.w = pack_t<TX>(q[6], q[7]);
+    r.x = pack2<TX>(q[0], q[1]);
+    r.y = pack2<TX>(q[2], q[3]);
+    r.z = pack2<TX>(q[4], q[5]);
+    r.w = pack2<TX>(q[6], q[7]);
     return r;
 }
 

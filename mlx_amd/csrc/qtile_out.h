@@ -15,16 +15,6 @@ typedef uint32_t t4 __attribute__((ext_vector_type(4), aligned(16)));
 constexpr int kCUs = 256;
 constexpr size_t kTileBytes = 128 * 1024;  // both GEMMs' tiles hold 32 Ki fp32 sums
 
-// two fp32 values -> a packed pair of T, RNE
-template <int T>
-__device__ __forceinline__ uint32_t pair(float a, float b) {
-    typedef float f2 __attribute__((ext_vector_type(2)));
-    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    if constexpr (T == DT_BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, b2));
-    else return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, h2));
-}
-
 // 8 columns n .. n + 7 of rows of y, through the output stage: their biases,
 // loaded once, and one (16-bit y) or two (f32) 16-byte stores per row.  Rows
 // of any N and y of any alignment its type allows: the stores need no more
@@ -69,10 +59,10 @@ struct RowOut {
         u16x8 p;
         if (ep.out_dt == DT_BF16) {
 #pragma unroll
-            for (int e = 0; e < 8; e += 2) p[e / 2] = pair<DT_BF16>(o[e], o[e + 1]);
+            for (int e = 0; e < 8; e += 2) p[e / 2] = pack2<DT_BF16>(o[e], o[e + 1]);
         } else {
 #pragma unroll
-            for (int e = 0; e < 8; e += 2) p[e / 2] = pair<DT_F16>(o[e], o[e + 1]);
+            for (int e = 0; e < 8; e += 2) p[e / 2] = pack2<DT_F16>(o[e], o[e + 1]);
         }
         uint16_t* d = static_cast<uint16_t*>(y) + at;
         if (n + 8 <= N) {
