@@ -1,10 +1,11 @@
 """Launches issued back to back on the context stream with no host
 synchronization between them -- the pattern the benchmark times.
 
-The GEMMs that split work across blocks keep tile counters and flags in the
-context's workspace: the split last round of both large GEMMs (halves meet
-by the launch's epoch; counters never reset), the register-W GEMM's K parts
-and the split-K small-M GEMM (counters the last block returns to zero).
+The GEMMs that split work across blocks meet in the context's workspace: the
+split last round of both large GEMMs (halves meet by the launch's epoch;
+counters never reset), their K parts (partial tiles a second launch adds), and
+the split-K small-M GEMM and the group-wise GEMM (counters the last block
+returns to zero).
 Each case here uploads its inputs once, enqueues LAUNCHES launches into
 separate output buffers without a synchronize, synchronizes once, then
 checks launch 0 against the oracle and every later launch bit for bit
@@ -28,8 +29,14 @@ LAUNCHES = 8
 CASES = [
     # configs[3] N = 14336: 896 tiles, the last 128 as two K halves each
     ("c3_n14336_split_last_round", (2048, 4096, 14336, 4, 64, BF16, BF16, BF16, 0), True, "qgemm_rw_kernel"),
-    # 128 tiles of 128 x 256, each in two K parts
-    ("rw_k_parts", (1024, 4096, 4096, 4, 64, BF16, BF16, F32, 2), True, "qgemm_rw_kernel"),
+    # 64 tiles of 128 x 256, each in 4 K parts
+    ("rw_k_parts", (512, 4096, 4096, 4, 64, BF16, BF16, F32, 2), True, "qgemm_rw_kernel"),
+    # 128 tiles of 128 x 256, each as two K halves
+    ("rw_all_tiles_split", (1024, 4096, 4096, 4, 64, BF16, BF16, F32, 2), True, "qgemm_rw_kernel"),
+    # 64 tiles of 256 x 128, each in 4 K parts
+    ("gemm_k_parts", (512, 4096, 4096, 3, 64, BF16, BF16, F32, 2), True, "qgemm_kernel"),
+    # 32 tiles of 64 x 128, each in 8 K parts the last of which adds them all
+    ("group_k_parts", (64, 4096, 4096, 4, 64, F32, F32, F32, 0), False, "qgemm_grp_kernel"),
     # 3-bit codes: the LDS-dequant GEMM, 128 tiles of 256 x 128, every one
     # as two K halves
     ("gemm_all_tiles_split", (1024, 4096, 4096, 3, 64, BF16, BF16, F32, 2), True, "qgemm_kernel"),

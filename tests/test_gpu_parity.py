@@ -787,14 +787,14 @@ def test_config3_prefill(ctx, oracle, N):
 
 def test_gemm_split_last_round(ctx, oracle):
     """The large GEMM runs a last round that is at most half full as two K
-    halves per tile, meeting in the context's workspace: 16 tiles (all
+    halves per tile, meeting in the context's workspace: 88 tiles (all
     split), then 264 tiles (the last 8 split: one column of tiles, all M
     tiles), then the first shape again.  Each tile counter must be back at
     zero after its launch, and a split result equals the oracle's
     dequantize-to-bf16 form as the unsplit tiles do; the first shape's
     repeat is bit-identical to its first run."""
     O = oracle
-    A = (512, 1024, 1024)
+    A = (1024, 1024, 2816)
     B = (2048, 512, 4224)
     first = None
     for i, (M, K, N) in enumerate([A, B, A]):
@@ -865,20 +865,34 @@ FUSED_CASES = [
     (3, 5120, 40, 5, 64, BF16),     # split-K GEMV on pairs of rows (5-bit, three rows of x)
     (3, 14336, 72, 4, 64, F16),     # 4x4x4-MFMA decode, two chunks per lane
     (6, 11008, 72, 4, 64, BF16),    # rows 0..3 and 4..5 as two launches (two-chunk decode)
-    (2, 4096, 40, 4, 64, F16),      # K-split whole-line GEMV (two rows of x)
+    (2, 4096, 40, 4, 64, F16),      # 4x4x4-MFMA decode (two rows of x)
     (2, 4096, 40, 3, 64, F16),      # stream GEMV (two rows of x, 3-bit)
     (6, 960, 70, 3, 64, F16),       # stream GEMV in chunks of 4 rows (3-bit, K % 1024 != 0)
     (3, 1024, 50, 6, 64, F32),      # whole-line GEMV once per row (f32 x, 6-bit)
     (6, 512, 96, 4, 64, BF16),      # skinny MFMA GEMV
     (3, 1024, 72, 8, 128, BF16),    # K-split whole-line GEMV (three rows of x, 8-bit)
-    (6, 4096, 64, 4, 64, BF16),     # decode MFMA kernel
-    (6, 2048, 40, 8, 128, F16),     # mid-M ring kernel (8-bit)
+    (6, 4096, 64, 4, 64, BF16),     # 4x4x4-MFMA decode (six rows of x)
+    (3, 1024, 40, 4, 64, F16),      # decode MFMA kernel
+    (6, 2048, 40, 8, 128, F16),     # skinny MFMA GEMV (8-bit)
+    (9, 1024, 40, 8, 128, F16),     # mid-M ring kernel (8-bit)
     (32, 2048, 72, 4, 64, BF16),    # small-M GEMM
     (24, 1024, 8300, 3, 64, F16),   # small-M GEMM, two column tiles per block (N > 8192)
     (40, 2560, 200, 4, 64, F16),    # split-K small-M GEMM (7 K parts)
     (96, 512, 136, 4, 64, F16),     # large GEMM
     (3, 96, 20, 4, 32, F32),        # generic kernel (K % 64 != 0)
+    (20, 1024, 130, 4, 64, F32),    # group-wise GEMM, f32 x, one 32-row tile, K parts
+    (70, 960, 300, 3, 64, BF16),    # group-wise GEMM, 16-bit x, two 64-row tiles, K % 128 == 64
+    (40, 4160, 300, 4, 64, F16),    # group-wise GEMM, 16-bit x, 16 K parts
+    (33, 640, 1001, 5, 32, F32),    # group-wise GEMM, f32 x, odd N
+    (100, 14336, 1003, 8, 64, F16),  # register-W GEMM, 4 tiles in 28 K parts, odd N
 ]
+# the kernel of each
+FUSED_KERNELS = 2 * ["qgemv_line_kernel"] + 2 * ["qgemv_split_kernel"] + [
+    "qgemv_q4_kernel", "qgemv_q4_kernel", "qgemv_q4_kernel", "qgemv_stream_kernel", "qgemv_stream_kernel",
+    "qgemv_line_kernel", "qmm_skinny_kernel", "qgemv_mx_kernel", "qgemv_q4_kernel", "qgemv_dec_kernel",
+    "qmm_skinny_kernel", "qgemv_mid_kernel", "qgemm_small_kernel", "qgemm_small_kernel", "qgemm_sk_kernel",
+    "qgemm_kernel", "qmm_generic_kernel"] + \
+    4 * ["qgemm_grp_kernel"] + ["qgemm_rw_kernel"]
 
 
 @pytest.mark.parametrize("case", FUSED_CASES, ids=lambda c: f"M{c[0]}K{c[1]}N{c[2]}b{c[3]}")
@@ -892,6 +906,7 @@ def test_fused_bias_activation(ctx, oracle, case, act):
     O = oracle
     M, K, N, bits, gs, xd = case
     sbd = F16 if xd == F32 else xd
+    assert ctx.kernel_name(M, K, N, gs, bits, xd, sbd, F32) == FUSED_KERNELS[FUSED_CASES.index(case)]
     x, w_q, s, b, _ = O.make_problem(M, K, N, bits, gs, xd, sbd, seed=5000 + M + act)
     bias_dt = [F32, F16, BF16, F32][act]
     bias = O.from_f32(O.rng_normal(N, seed=6000 + N), bias_dt)
@@ -1156,6 +1171,39 @@ def test_lds_gemm_k_parts(ctx, oracle, bits, M, K, N, gs, xd, sbd, od, act):
             0.5 * want * (1 + np.vectorize(erf)(want / np.sqrt(2.0)))
     check_output(O, np.ascontiguousarray(ys[0][rows]), O.from_f32(want.astype(np.float32), od), od,
                  f"K parts b{bits} M{M} K{K} N{N}")
+
+
+@pytest.mark.parametrize("M,K,N,bits,gs,xd,sbd,od,act", [
+    (300, 11264, 2100, 4, 64, F16, F16, F16, 3),   # 27 tiles, 22 loops in 8 parts, GELU
+    (700, 5120, 2101, 8, 128, BF16, F16, F32, 0),  # 54 tiles, 5 loops in 3 parts, odd N
+    (300, 5120, 2101, 4, 32, F16, BF16, BF16, 2)])  # 27 tiles, 20 loops in 7 parts, SiLU, odd N
+def test_rw_gemm_uneven_k_parts(ctx, oracle, M, K, N, bits, gs, xd, sbd, od, act):
+    """The register-W GEMM in K parts of different lengths summed by a second
+    launch, with the fused output stage there, twice (the same bits), against
+    the dequantize-to-T form."""
+    from mlx_amd import runtime
+    O = oracle
+    assert ctx.kernel_name(M, K, N, gs, bits, xd, sbd, od) == "qgemm_rw_kernel"
+    x, w_q, s, b, _ = O.make_problem(M, K, N, bits, gs, xd, sbd, seed=8350 + M + bits)
+    rows = np.unique(np.r_[0, M // 3, M - 1])
+    acc = O.quantized_matmul(np.ascontiguousarray(x[rows]), w_q, s, b, len(rows), K, N, gs, bits, xd, sbd, F32,
+                             variant="omp", w_round=xd)
+    bias = O.rng_normal(N, seed=8450 + N).astype(np.float32)
+    bufs = [ctx.upload(a) for a in (x, w_q, s, b)]
+    bb = ctx.upload(bias)
+    out = ctx.alloc(M * N * runtime.esize(od))
+    try:
+        ys = []
+        for _ in range(2):
+            print(f"[case] rw K parts M={M} K={K} N={N} b{bits} act={act}", flush=True)
+            ctx.quantized_matmul_fused(*bufs, bb if act else None, out, M, K, N, gs, bits, xd, sbd, F32, od, act)
+            ys.append(out.download(runtime.np_dtype(od), (M, N)))
+    finally:
+        for t in bufs + [bb, out]:
+            t.free()
+    assert np.array_equal(ys[0], ys[1])
+    want = O.fused_epilogue(acc, bias if act else None, F32, act, od)
+    check_output(O, np.ascontiguousarray(ys[0][rows]), want, od, f"rw K parts b{bits} M{M} K{K} N{N}")
 
 
 @pytest.mark.parametrize("bits", BITS)

@@ -22,7 +22,7 @@ the oracle checks of these kernels are in test_gpu_parity.py.
 
 The GEMMs get the same check over scale dtype x group size (which set the
 register-W GEMM's scale windows, unroll and compile-time wait counts): the
-register-W GEMM with K parts meeting in the workspace and on its persistent
+register-W GEMM with K parts or halves meeting in the workspace and on its persistent
 grid with a split last round, the split-K small-M GEMM (K parts, counters
 the last part returns to zero) and the LDS-dequant GEMM for the other code
 widths.  So do the GEMV kernels AUTO picks for M = 1..8.
@@ -110,8 +110,9 @@ def test_mid_gemv_rings_repeat(ctx, bits, sbd):
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("sbd", SB, ids=["sb_f16", "sb_bf16", "sb_f32"])
 def test_rw_gemm_repeat(ctx, bits, sbd):
-    """qgemm_rw, every group size: 30 tiles in K parts meeting in the
-    workspace (M = 640, N = 1536, fp32 out), and 264 tiles on the persistent
+    """qgemm_rw, every group size: 30 tiles in 4 K parts (two halves with 16-bit
+    scales of groups of 128) meeting in the workspace (M = 640, N = 1536, fp32
+    out), and 264 tiles on the persistent
     grid, the last round's 8 tiles in K halves (M = 1024, N = 8448, 16-bit
     out); K = 2048."""
     xd = BF16 if sbd == BF16 else F16

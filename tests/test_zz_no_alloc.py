@@ -5,10 +5,12 @@ kernels, and the same K split, since its static scratch is the size of a
 context's workspace), and within the output gate of the oracle.  Two calls
 in a row share the scratch, the second with a smaller input; the first two
 run the split-K GEMM with its parts meeting in the scratch, the next two the
-large GEMM with the two K halves of its tiles meeting there, so a counter or
+large GEMMs with the two K halves of their tiles meeting there, so a counter or
 flag left nonzero by one call would break the next; the fifth runs the large
 GEMM on one block per CU (more tiles than CUs, 16-bit output), its blocks
-going on from a whole tile to a K half.
+going on from a whole tile to a K half; the sixth and seventh K parts of the
+large GEMM, summed by a second launch, and of the group-wise GEMM, summed by
+the last to arrive.
 """
 import ctypes
 import os
@@ -24,9 +26,11 @@ pytestmark = pytest.mark.gpu
 CALLS = [
     (64, 3584, 4096, 3, 64, F16, F16, F16, 0),     # split-K GEMM, 4 K parts, 128 blocks
     (17, 1152, 200, 4, 32, BF16, BF16, F32, 2),    # split-K GEMM, 3 K parts, 6 blocks
-    (512, 1024, 1024, 4, 64, BF16, BF16, F32, 2),  # large GEMM, 16 tiles, each in two K halves
-    (300, 512, 200, 4, 64, F16, F16, F16, 2),      # large GEMM, 4 ragged tiles, each in two K halves
+    (1024, 1024, 2816, 4, 64, BF16, BF16, F32, 2),  # register-W GEMM, 88 tiles, each in two K halves
+    (600, 1024, 1500, 3, 64, F16, F16, F16, 2),    # LDS-dequant GEMM, 36 ragged tiles, each in two K halves
     (2000, 1024, 4360, 4, 64, BF16, BF16, BF16, 2),  # large GEMM, one block per CU: 288 ragged tiles, 32 in K halves
+    (300, 512, 200, 4, 64, F16, F16, F16, 2),      # LDS-dequant GEMM, 4 ragged tiles in 2 K parts
+    (40, 4160, 300, 4, 64, F32, F32, F32, 0),      # group-wise GEMM, 3 tiles in 16 K parts
     (1, 4096, 512, 4, 64, F16, F16, F16, 0),       # a GEMV: no scratch
 ]
 
@@ -101,7 +105,7 @@ def test_noalloc_matches_context_op(ctx, oracle):
 
 
 def test_noalloc_back_to_back(ctx, oracle):
-    """The split-K, split-last-round and persistent calls of CALLS enqueued
+    """The split-K, split-last-round, persistent and K-part calls of CALLS enqueued
     on one stream with no synchronize between them (the scratch's counters
     and flags must be back at zero when the next call starts), then each
     output against the context op on the same inputs, bit for bit."""
@@ -111,11 +115,11 @@ def test_noalloc_back_to_back(ctx, oracle):
     hip = _Hip()
     stream = ctypes.c_void_p()
     hip.ck(hip.L.hipStreamCreate(ctypes.byref(stream)), "hipStreamCreate")
-    calls, held = CALLS[:5] * 2, []
+    calls, held = CALLS[:7] * 2, []
     try:
         for i, (M, K, N, bits, gs, xd, sbd, od, kern) in enumerate(calls):
             print(f"[case] noalloc back-to-back call {i}: M={M} K={K} N={N} b={bits} kernel={kern}", flush=True)
-            x, w_q, s, b, _ = O.make_problem(M, K, N, bits, gs, xd, sbd, seed=700 + i % 5)
+            x, w_q, s, b, _ = O.make_problem(M, K, N, bits, gs, xd, sbd, seed=700 + i % 7)
             ptrs = [hip.upload(np.ascontiguousarray(a)) for a in (x, w_q, s, b)]
             out = hip.alloc(M * N * runtime.esize(od))
             held.append((ptrs, out, (x, w_q, s, b), (M, K, N, bits, gs, xd, sbd, od, kern)))
