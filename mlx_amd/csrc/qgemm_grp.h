@@ -10,8 +10,8 @@
 //    exactly: its leading 8 significant bits, the next 8 and the last 8, each
 //    by truncation (so the first never rounds up to infinity).  Below 2^-109
 //    the third underflows: a tile with a row of x that has nothing from 2^-100
-//    on is run once more, with such rows times 2^24 (watching for them costs 2 %
-//    of M = 64, K = N = 4096, 4-bit: 21.2 against 21.6 us);
+//    on is run once more, with such rows times 2^24 (watching for them costs 1 to
+//    2 %: M = 64, K = N = 4096, 4-bit 19.8 against 20.0 us);
 //  * a product of the two has at most 19 bits and is exact in the f32
 //    accumulator, which is started afresh for every group and then scaled
 //    into the f32 sums of y.
@@ -87,10 +87,11 @@ struct Lds {
     static constexpr int kScales = kCodes + 2 * BN * kCodeRow;
     static constexpr int kOut = BN + 4;                    // floats per row of the output tile
     static constexpr int kTile = BM * kOut * 4;            // two of them at the end (pairs of K parts)
-    static constexpr int kRows = 2 * kTile;                // past the tiles: 8 flags, then a value per row
-    static constexpr int kEnd = kRows + 32 + 4 * BM;
+    static constexpr int kRows = 2 * kTile;                // past the tiles: a value per row
+    static constexpr int kEnd = kRows + 4 * BM;
     static constexpr int kLoop = kScales + 2 * kWindow;
-    static constexpr int kBytes = kLoop > kEnd ? kLoop : kEnd;
+    static constexpr int kFlag = kLoop > kEnd ? kLoop : kEnd;  // past all of that: a word
+    static constexpr int kBytes = kFlag + 16;
     static_assert(kBytes <= 160 * 1024, "LDS");
 };
 
@@ -150,12 +151,12 @@ constexpr float kSmall = 0x1p-100f, kSmallUp = 0x1p24f, kSmallDown = 0x1p-24f;
 // One run over steps s0 .. s1 - 1 of the tile at (m0, n0): its sums in o.
 // BITS: code width; TX: type of x; SBF: f32 scales (else 16-bit ones, sb_dt
 // says which); MT: 32-row tiles.  f32 x: true where a row has nothing from
-// kSmall on; again then takes such rows times kSmallUp (bit i of small: the
+// kSmall on; run 1 then takes such rows times kSmallUp (bit i of small: the
 // thread's load i of x is of one, of rows: its vector i of the output).
 template <int BITS, int TX, bool SBF, int MT>
 __device__ __forceinline__ bool run_tile(uint8_t* lds, const void* __restrict__ x, const uint32_t* __restrict__ wq,
                                          const void* __restrict__ scales, const void* __restrict__ biases, int M, int K,
-                                         int N, int gshift, int sb_dt, int m0, int n0, int s0, int s1, bool again,
+                                         int N, int gshift, int sb_dt, int m0, int n0, int s0, int s1, int run,
                                          uint32_t& small, uint32_t& rows, f4 (&o)[kOutVecs<MT>]) {
     constexpr int P = TX == DT_F32 ? 3 : 1;       // planes of x
     using L = Lds<MT, BITS, P>;
@@ -171,6 +172,8 @@ __device__ __forceinline__ bool run_tile(uint8_t* lds, const void* __restrict__ 
     int tid = threadIdx.x;
     // (addresses of a run are its own: kept over both they cost 80 registers)
     if constexpr (TX == DT_F32) asm volatile("" : "+v"(tid));
+    tid &= kThreads - 1;  // (what the compiler knew of it)
+    const bool again = __builtin_amdgcn_readfirstlane(run) != 0;  // (scalar branches)
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kg = wave >> 1, nw = wave & 1;
@@ -292,11 +295,14 @@ __device__ __forceinline__ bool run_tile(uint8_t* lds, const void* __restrict__ 
     };
 
     auto scale_x = [&](Raw& o) LXQ_INLINE {
+        uint32_t m = small;
+        asm volatile("" : "+v"(m));  // nothing of this in front of the branch to it
 #pragma unroll
-        for (int i = 0; i < XL; i++)
+        for (int i = 0; i < XL; i++) {
+            const float f = (m >> i) & 1u ? kSmallUp : 1.f;
 #pragma unroll
-            for (int e = 0; e < 4; e++)
-                if ((small >> i) & 1u) o.x[i][e] = __float_as_uint(__uint_as_float(o.x[i][e]) * kSmallUp);
+            for (int e = 0; e < 4; e++) o.x[i][e] = __float_as_uint(__uint_as_float(o.x[i][e]) * f);
+        }
     };
     uint32_t lost = 0;  // the third terms' bits of all steps
 
@@ -399,6 +405,8 @@ __device__ __forceinline__ bool run_tile(uint8_t* lds, const void* __restrict__ 
         __syncthreads();
     };
 
+    uint32_t* flag = reinterpret_cast<uint32_t*>(lds + L::kFlag);
+    if (TX == DT_F32 && tid == 0) *flag = 0u;
     Raw next;
     {
         float sum[XL];
@@ -421,11 +429,7 @@ __device__ __forceinline__ bool run_tile(uint8_t* lds, const void* __restrict__ 
     // 32 x 32 tile, register v its row 8 (v / 4) + 4 h + v % 4): parts 0 and 2
     // store, 1 and 3 add theirs
     float* ot = reinterpret_cast<float*>(lds + (kg >> 1) * L::kTile);
-    uint32_t* flags = reinterpret_cast<uint32_t*>(lds + L::kRows);
-    if constexpr (TX == DT_F32) {
-        const bool any = __any((lost & 0xffffu) != 0u);
-        if (lane == 0) flags[wave] = any ? 1u : 0u;
-    }
+    if (TX == DT_F32 && (lost & 0xffffu) != 0u) *flag = 1u;
 #pragma unroll
     for (int half = 0; half < 2; half++) {
         if ((kg & 1) == half) {
@@ -446,12 +450,15 @@ __device__ __forceinline__ bool run_tile(uint8_t* lds, const void* __restrict__ 
     for (int i = 0; i < kOutVecs<MT>; i++) {
         const float* d = reinterpret_cast<const float*>(lds) + (orow + 16 * i) * L::kOut + oc;
         o[i] = *reinterpret_cast<const f4*>(d) + *reinterpret_cast<const f4*>(d + L::kTile / 4);
-        if (TX == DT_F32 && again && ((rows >> i) & 1u)) o[i] *= kSmallDown;
     }
     if constexpr (TX != DT_F32) return false;
-    if (again) return false;
-    const u4 f0 = *reinterpret_cast<const u4*>(flags), f1 = *reinterpret_cast<const u4*>(flags + 4), fa = f0 | f1;
-    if ((fa[0] | fa[1] | fa[2] | fa[3]) == 0u) return false;
+    if (again) {
+#pragma unroll
+        for (int i = 0; i < kOutVecs<MT>; i++)
+            if ((rows >> i) & 1u) o[i] *= kSmallDown;
+        return false;
+    }
+    if (__builtin_amdgcn_readfirstlane(*flag) == 0u) return false;
     // bits were lost somewhere (a tail of SiLU or of an exponential will do
     // it): the largest x of each row
     float most[XL];
@@ -464,7 +471,7 @@ __device__ __forceinline__ bool run_tile(uint8_t* lds, const void* __restrict__ 
 #pragma unroll
             for (int e = 0; e < 4; e++) most[i] = fmaxf(most[i], fabsf(__uint_as_float(next.x[i][e])));
     }
-    float* row_most = reinterpret_cast<float*>(flags + 8);
+    float* row_most = reinterpret_cast<float*>(lds + L::kRows);
 #pragma unroll
     for (int i = 0; i < XL; i++) {
 #pragma unroll
@@ -494,10 +501,9 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
     const int s0 = (int)((long long)steps * part / parts), s1 = (int)((long long)steps * (part + 1) / parts);
     f4 o[kVec];
     uint32_t small = 0, rows = 0;
-    bool again = false;
-    while (run_tile<BITS, TX, SBF, MT>(lds, x, wq, scales, biases, M, K, N, gshift, sb_dt, m0, n0, s0, s1, again, small,
-                                       rows, o))
-        again = true;
+    for (int run = 0; run_tile<BITS, TX, SBF, MT>(lds, x, wq, scales, biases, M, K, N, gshift, sb_dt, m0, n0, s0, s1,
+                                                  run, small, rows, o);)
+        run = 1;
     const int tid = threadIdx.x, oc = 4 * (tid & 31), orow = tid >> 5;
     constexpr uint32_t kSlot = BM * BN * 4;
     if (parts > 1) {
