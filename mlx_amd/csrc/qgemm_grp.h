@@ -10,8 +10,7 @@
 //    exactly: its leading 8 significant bits, the next 8 and the last 8, each
 //    by truncation (so the first never rounds up to infinity).  Below 2^-109
 //    the third underflows: a tile with a row of x that has nothing from 2^-100
-//    on is run once more, with such rows times 2^24 (watching for them costs 1 to
-//    2 %: M = 64, K = N = 4096, 4-bit 19.8 against 20.0 us);
+//    on is run once more, with such rows times 2^24;
 //  * a product of the two has at most 19 bits and is exact in the f32
 //    accumulator, which is started afresh for every group and then scaled
 //    into the f32 sums of y.
@@ -170,8 +169,11 @@ __device__ __forceinline__ bool run_tile(uint8_t* lds, const void* __restrict__ 
     constexpr int kSb = SBF ? 4 : 2;
     constexpr float C = (float)(1 << (BITS - 1));
     int tid = threadIdx.x;
-    // (addresses of a run are its own: kept over both they cost 80 registers)
-    if constexpr (TX == DT_F32) asm volatile("" : "+v"(tid));
+    // Each run works its addresses out anew: kept over both they cost 80
+    // registers, and worked out ahead of the loop around the runs they stood in
+    // front of the first load (M = 64, K = N = 4096, 4-bit: 20.5 us, so 19.7).
+    if constexpr (TX == DT_F32)
+        asm volatile("" : "+v"(tid), "+s"(M), "+s"(K), "+s"(N), "+s"(gshift), "+s"(m0), "+s"(n0), "+s"(s0), "+s"(s1));
     tid &= kThreads - 1;  // (what the compiler knew of it)
     const bool again = __builtin_amdgcn_readfirstlane(run) != 0;  // (scalar branches)
     const int lane = tid & 63;
@@ -187,6 +189,20 @@ __device__ __forceinline__ bool run_tile(uint8_t* lds, const void* __restrict__ 
 #pragma unroll
     for (int i = 0; i < XL; i++)
         xp[i] = static_cast<const uint8_t*>(x) + (size_t)min(m0 + xr + XR * i, M - 1) * K * (16 / XE);
+    struct Raw {
+        u4 x[XL];
+        u4 c[CL];
+    };
+    auto load_x = [&](Raw& o, int s) LXQ_INLINE {
+#pragma unroll
+        for (int i = 0; i < XL; i++)
+            o.x[i] = *reinterpret_cast<const u4h*>(xp[i] + (size_t)min(s * BK + XE * xc, K - XE) * (16 / XE));
+    };
+    // the first step's x, ahead of every other address (in the scheduler's
+    // order, behind all of them, 20.0 us there)
+    Raw next;
+    load_x(next, s0);
+    __builtin_amdgcn_sched_barrier(0);
     // codes: chunk q = t + 512 i of the block's 128 BITS: column q / BITS, 16
     // bytes q % BITS of its step (columns past N re-read the last; a half
     // step at the end of K reads on into the next row or the readable tail)
@@ -198,6 +214,11 @@ __device__ __forceinline__ bool run_tile(uint8_t* lds, const void* __restrict__ 
         cp[i] = reinterpret_cast<const uint8_t*>(wq) + (size_t)min(n0 + col, N - 1) * ((size_t)K * BITS / 8) + b;
         cd[i] = col * L::kCodeRow + b;
     }
+    auto load_codes = [&](Raw& o, int s) LXQ_INLINE {
+#pragma unroll
+        for (int i = 0; i < CL; i++) o.c[i] = *reinterpret_cast<const u4g*>(cp[i] + (size_t)s * (16 * BITS));
+    };
+    load_codes(next, s0);
     // scales: thread t loads 16 bytes (half t / 256) of the window of column t
     // % 128, scales or biases (t / 128 % 2); a window is 32 / kSb groups
     const int gws = 5 - (SBF ? 2 : 1) + gshift - 7;  // steps per window, log2
@@ -212,16 +233,9 @@ __device__ __forceinline__ bool run_tile(uint8_t* lds, const void* __restrict__ 
         for (int e = 0; e < 4; e++) d[e] = v[e];
     };
 
-    struct Raw {
-        u4 x[XL];
-        u4 c[CL];
-    };
     auto load = [&](Raw& o, int s) LXQ_INLINE {
-#pragma unroll
-        for (int i = 0; i < XL; i++)
-            o.x[i] = *reinterpret_cast<const u4h*>(xp[i] + (size_t)min(s * BK + XE * xc, K - XE) * (16 / XE));
-#pragma unroll
-        for (int i = 0; i < CL; i++) o.c[i] = *reinterpret_cast<const u4g*>(cp[i] + (size_t)s * (16 * BITS));
+        load_x(o, s);
+        load_codes(o, s);
     };
     auto store_codes = [&](const Raw& o, int stage) LXQ_INLINE {
         uint8_t* d = lds + L::kCodes + stage * (BN * L::kCodeRow);
@@ -407,11 +421,9 @@ __device__ __forceinline__ bool run_tile(uint8_t* lds, const void* __restrict__ 
 
     uint32_t* flag = reinterpret_cast<uint32_t*>(lds + L::kFlag);
     if (TX == DT_F32 && tid == 0) *flag = 0u;
-    Raw next;
     {
         float sum[XL];
         uint32_t low = 0;
-        load(next, s0);
         const u4 w0 = load_win(s0 >> gws);
         if (TX == DT_F32 && again) scale_x(next);
 #pragma unroll
@@ -492,13 +504,16 @@ template <int BITS, int TX, bool SBF, int MT>
 __global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
     const void* __restrict__ x, const uint32_t* __restrict__ wq, const void* __restrict__ scales,
     const void* __restrict__ biases, void* __restrict__ y, int M, int K, int N, int gshift, int sb_dt, Epilogue ep,
-    int mtiles, int tiles, int parts, void* __restrict__ ws) {
+    int mtiles, int each, int longer, void* __restrict__ ws) {
     constexpr int BM = 32 * MT, kVec = kOutVecs<MT>;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    const int tile = (int)blockIdx.x % tiles, part = (int)blockIdx.x / tiles;
-    const int m0 = tile % mtiles * BM, n0 = tile / mtiles * BN;
-    const int steps = (K + BK - 1) / BK;
-    const int s0 = (int)((long long)steps * part / parts), s1 = (int)((long long)steps * (part + 1) / parts);
+    // grid: (tiles, parts); the first `longer` parts are each + 1 steps
+    // (no divisions where there is one tile of rows: the first loads wait for
+    // all of this)
+    const int tile = (int)blockIdx.x, part = (int)blockIdx.y;
+    const unsigned un = mtiles == 1 ? blockIdx.x : blockIdx.x / (unsigned)mtiles;
+    const int m0 = (int)(blockIdx.x - un * (unsigned)mtiles) * BM, n0 = (int)un * BN;
+    const int s0 = part * each + min(part, longer), s1 = s0 + each + (part < longer ? 1 : 0);
     f4 o[kVec];
     uint32_t small = 0, rows = 0;
     for (int run = 0; run_tile<BITS, TX, SBF, MT>(lds, x, wq, scales, biases, M, K, N, gshift, sb_dt, m0, n0, s0, s1,
@@ -506,6 +521,7 @@ __global__ __launch_bounds__(kThreads, 1) void qgemm_grp_kernel(
         run = 1;
     const int tid = threadIdx.x, oc = 4 * (tid & 31), orow = tid >> 5;
     constexpr uint32_t kSlot = BM * BN * 4;
+    const int tiles = (int)gridDim.x, parts = (int)gridDim.y;
     if (parts > 1) {
         const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(
             static_cast<uint8_t*>(ws) + split::kPartOffset, 0, (int)((uint32_t)(tiles * parts) * kSlot), 0x00020000);
@@ -583,8 +599,9 @@ LuxStatus launch_t(const QmmArgs& a, hipStream_t st) {
         if (parts < 1) parts = 1;
     }
     const int gshift = a.group_size == 32 ? 5 : a.group_size == 64 ? 6 : 7;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * parts)), dim3(kThreads), L::kBytes, st, a.x, a.wq, a.scales,
-                       a.biases, a.y, a.M, a.K, a.N, gshift, a.sb_dtype, a.epi(), mtiles, tiles, parts, a.ws);
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)parts), dim3(kThreads), L::kBytes, st, a.x, a.wq, a.scales,
+                       a.biases, a.y, a.M, a.K, a.N, gshift, a.sb_dtype, a.epi(), mtiles, steps / parts, steps % parts,
+                       a.ws);
     return hipGetLastError() == hipSuccess ? LuxStatus::Ok : LuxStatus::Internal;
 }
 
