@@ -54,9 +54,9 @@ __global__ __launch_bounds__(256) void ew_kernel(const float* __restrict__ a, co
 // read per row or column and 4 k.
 //
 // Bound by VALU issue (32-bit multiply and add, packed forms excluded): 55
-// TFLOP/s at 2048^3 and 44 at 1000 x 2000 x 3000 (272 us), where one
-// multiply-add pair per lane and 4 clocks would be 39 and two 78.  4 x 4 tiles
-// read from LDS word by word, k by k, took 474 us there.
+// TFLOP/s at 2048^3 and 40 to 43 at 1000 x 2000 x 3000 (281 to 298 us by box),
+// where one multiply-add pair per lane and 4 clocks would be 39 and two 78.
+// 4 x 4 tiles read from LDS word by word, k by k, took 474 us there.
 template <int TM_, int TN_, int RM_, int RN_, int TK_, int KM_>
 struct MmTile {
     static constexpr int TM = TM_, TN = TN_, RM = RM_, RN = RN_, TK = TK_, KM = KM_;
