@@ -45,7 +45,8 @@
 //
 // K is split over `parts` blocks per tile where the tiles alone would leave
 // CUs idle; the parts' tiles meet in the workspace (qsplit.h, K parts), where
-// the last to arrive adds all of them in part order.
+// the last to arrive adds all of them in part order, four at a time as two
+// pairs.
 #pragma once
 #include <type_traits>
 
